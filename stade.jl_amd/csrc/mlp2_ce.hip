@@ -1099,13 +1099,6 @@ __global__ __launch_bounds__(NT) void final_kernel(FinalArgs f) {
     final_block<MODE>(f, blockIdx.x, red);
 }
 
-// resident blocks per CU of the adjoint's paired backward launch (its registers would allow
-// four; three measured faster)
-#ifndef STADE_MLP_BWD_BLOCKS
-#define STADE_MLP_BWD_BLOCKS 3
-#endif
-constexpr int kBwdBlocksPerCu = STADE_MLP_BWD_BLOCKS;
-
 // the final sums as extra blocks of the backward products' launch (they read only the head
 // and column-sum partials, so they run beside the product tiles)
 template <int MODE>
@@ -1172,8 +1165,11 @@ int32_t run(const Ptrs& p, int64_t B_, int64_t I_, int64_t H_, int64_t O_, hipSt
     // products: one launch each, operand tiles shared)
     const Plan p_s1 = plan(H, B, I, cus), p_s1d = plan(H, B, I, cus, 2);
     // (the backward products only accumulate into shadows: their K splits may add by atomics)
-    const Plan p_w1b = plan(H, I, B, cus, 1, true), p_w1bd = plan(H, I, B, cus, 2, true);
-    const Plan p_xb = plan(I, B, H, cus, 1, true), p_xbd = plan(I, B, H, cus, 2, true);
+    // (and they run as one launch, so with one tile width)
+    const Plan p_w1bd = plan(H, I, B, cus, 2, true), p_xbd = plan(I, B, H, cus, 2, true);
+    auto both = [&](int bnt) { return std::pair<Plan, Plan>(plan(H, I, B, cus, 1, true, bnt), plan(I, B, H, cus, 1, true, bnt)); };
+    const auto n64 = both(64), n128 = both(128);
+    const auto& [p_w1b, p_xb] = n64.first.us + n64.second.us <= n128.first.us + n128.second.us ? n64 : n128;
     size_t npart = 0;
     auto need = [&](const Plan& q, long M, long N) {
         if (q.ksplit > 1) npart = std::max(npart, (size_t)q.ksplit * M * N);
@@ -1290,7 +1286,7 @@ int32_t run(const Ptrs& p, int64_t B_, int64_t I_, int64_t H_, int64_t O_, hipSt
             gw.nseg = gx.nseg = 1;
             STADE_TIMED("mlp_gemm_bwd", stream,
                         e = (launch_pair<false, false, EpiAcc, true, true, EpiAcc>(gw, EpiAcc{p.w1b, H}, p_w1b, gx, EpiAcc{p.xb, I},
-                                                                                   p_xb, stream, fin, kBwdBlocksPerCu)));
+                                                                                   p_xb, stream, fin)));
         } else {
             gw.seg[1] = Seg{D1d, p.xd, H, I, B};     // A1 = d1d, B1 = xd'
             gx.seg[1] = Seg{p.w1d, D1d, H, H, H};    // A1 = W1d', B1 = d1d

@@ -1,0 +1,85 @@
+"""The fp32 matrix products' split-bf16 form (csrc/gemm_f32.hpp) at the places where it can go
+wrong, through the MLP entry points: K of a partial step only, of whole steps only and of both,
+output tiles with one row or column past a tile's edge; operands that the split cannot hold
+(under 2^-110), whose tiles are formed again in fp32; and operands that are not finite or
+round to infinity in bf16.  The bar is the fp32 one (1e-5 normwise against the Float32 oracle,
+with the truth rule); the split's own error is at most 2^-24 of a product."""
+import numpy as np
+import pytest
+
+from helpers import ParityCase, make_args, oracle_lib, rel_err, run_parity, to_host
+
+pytestmark = pytest.mark.gpu
+
+
+def _shapes(size):
+    B, I, H, O = size
+    sz = dict(loss=1, x=I * B, w1=H * I, b1=H, w2=O * H, b2=O, h1=H * B, z=O * B)
+    return {k + suf: v for k, v in sz.items() for suf in ("", "b", "d", "bd")}
+
+
+def _labels(size):
+    return np.arange(size[0], dtype=np.int64) % size[3] + 1
+
+
+def _scales(size):
+    B, I, H, O = size
+    g1, g2 = np.sqrt(2.0 / (I + H)), np.sqrt(2.0 / (H + O))
+    return {"w1": g1, "w1d": g1, "w2": g2, "w2d": g2, "b1": 0.1, "b2": 0.1}
+
+
+def _ints(size):
+    return dict(zip(("i_b", "i_in", "i_h", "i_out"), size))
+
+
+@pytest.mark.parametrize("mode", ["b", "d", "hv"])
+@pytest.mark.parametrize("size", [(1, 1, 1, 1), (129, 15, 65, 5), (64, 16, 128, 5), (127, 17, 129, 3), (128, 48, 64, 4),
+                                  (161, 33, 97, 2)])
+def test_split_product_edges(mode, size):
+    print(f"mlp2_ce_{mode} {size}", flush=True)
+    run_parity("mlp2_ce", mode, _shapes(size), _ints(size), precision="f32", int_arrays=dict(lab=_labels(size)),
+               scales=_scales(size))
+
+
+@pytest.mark.parametrize("mode", ["b", "d", "hv"])
+def test_split_product_tiny_operands(mode):
+    """x and its direction near 2^-122, below what three bf16 values hold, against weights
+    near 2^110: every product is of ordinary size."""
+    size = (150, 40, 70, 6)
+    s = _scales(size)
+    for a in ("x", "xd"):
+        s[a] = 2.0 ** -122
+    for a in ("w1", "w1d"):
+        s[a] *= 2.0 ** 110
+    print(f"mlp2_ce_{mode} tiny operands", flush=True)
+    run_parity("mlp2_ce", mode, _shapes(size), _ints(size), precision="f32", int_arrays=dict(lab=_labels(size)), scales=s)
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan, 3.4e38])
+def test_split_product_non_finite(value):
+    """One element of x that is not finite, or whose nearest bf16 is infinite (with weights that
+    keep its products finite): the same elements of every output are finite as in the oracle,
+    the others agree in kind, and the finite ones to the fp32 bar."""
+    size = (140, 20, 130, 3)
+    s = _scales(size)
+    if np.isfinite(value):
+        s["w1"] *= 1e-30
+    lib = oracle_lib("mlp2_ce", "b", "f32")
+    args = make_args(lib, "mlp2_ce_b", _shapes(size), _ints(size), {}, "split-non-finite", np.float32, dict(lab=_labels(size)), s)
+    x = next(v for a, _, v in args if a == "x")
+    x[7 * size[1] + 3] = value
+    host = [v.copy() if isinstance(v, np.ndarray) else v for _, _, v in args]
+    lib.call("mlp2_ce_b", *host)
+    case = ParityCase("mlp2_ce", "b", args, (), "f32")
+    print(f"mlp2_ce_b one element {value}", flush=True)
+    case.run_gpu()
+    for (a, kind, _), want, dev in zip(args, host, case.dev):
+        if kind != "Af":
+            continue
+        got = to_host(dev)
+        assert np.array_equal(np.isnan(got), np.isnan(want)), a
+        inf = np.isinf(want)
+        assert np.array_equal(np.isinf(got), inf) and np.array_equal(got[inf], want[inf]), a
+        ok = np.isfinite(want)
+        if np.any(want[ok]):
+            assert rel_err(got[ok], want[ok]) <= 1e-5, a
