@@ -13,8 +13,8 @@
 //   adjoint  g = outb + (0.5 (2 out)) lossb  (the accumulated outb, then reset to 0)
 //            wb[co][c][ky][kx] += sum_{n,y,x} g[n][co][y][x] xp[n][c][y+ky][x+kx]
 //            xpb[n][c][yp][xq] += sum_{co,ky,kx} w[co][c][ky][kx] g[n][co][yp-ky][xq-kx]
-// All three run on the fp32 matrix cores (v_mfma_f32_32x32x2_f32) as implicit GEMMs: no
-// im2col buffer; each block stages an input patch and a weight slice in LDS and the MFMA
+// All three run on the matrix cores as implicit GEMMs (the tap kernel's by split bf16, the
+// weight gradient's by v_mfma_f32_32x32x2_f32): no im2col buffer; each block stages an input patch and a weight slice in LDS and the MFMA
 // operands are read from the patch at tap-shifted offsets.
 //   tap_kernel    forward (and the tangent's two products) and the interior of xpb, which
 //                 is the same shifted product on g with flipped, transposed weights
@@ -23,63 +23,107 @@
 //   wgrad_kernel  split over pixel tiles, partial 9 x 64 x 64 weight gradients per block
 //   wreduce_kernel sums the partials in a fixed order into wb
 #include "internal.hpp"
+#include "gemm_f32.hpp"
+#include "split_bf16.hpp"
 
 #include <algorithm>
 
 namespace stade {
 namespace {
 
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr int NT = 256;
 constexpr int kBufWord3 = 0x00020000;  // gfx9-family buffer resource word 3 (raw, 32-bit data)
-
-enum { FWD_B, FWD_D, FWD_HV, DG_B, DG_HV };
 
 __device__ __forceinline__ floatx16 mfma(float a, float b, floatx16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
+// 16-channel chunks of the tap kernel's input channels
+__host__ __device__ __forceinline__ int tap_chunks(int Cin) { return (Cin + 15) / 16; }
+
 // ------------------------------------------------------------------------------------------
-// weight layouts for the tap kernel: wt[cin][t][r] (rows padded to a multiple of 64 with
-// zeros).  Forward: cin = c, r = co, t = 3 ky + kx.  Interior of xpb: cin = co, r = c, and
-// the tap flipped (t' = 8 - t), so both products read their source at (y + ky' - 1 + ...).
+// weights for the tap kernel, split into their bf16 parts (split_bf16.hpp) in the order of the
+// matrix-core fragments that read them: 16-byte cell
+//   ((((rt * chunks + ch) * 9 + t) * 3 + part) * 2 + i) * 64 + lane
+// holds rows r = 64 rt + 32 i + lane % 32, input channels 16 ch + 8 (lane / 32) + 0..7 of tap t
+// (zero past the last row or channel).  Forward: cin = c, r = co, t = 3 ky + kx.  Interior of
+// xpb: cin = co, r = c, and the tap flipped (t' = 8 - t), so both products read their source
+// at (y + ky' - 1 + ...).  Each block also writes whether it met a weight that the split cannot
+// hold (flags[block]).
 // ------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(NT) void prep_kernel(const float* __restrict__ w, int C, int K, float* __restrict__ wf,
-                                                  int Kpad, float* __restrict__ wg, int Cpad) {
-    const long nf = (long)C * 9 * Kpad, ng = wg ? (long)K * 9 * Cpad : 0;
+__global__ __launch_bounds__(NT) void prep_kernel(const float* __restrict__ w, int C, int K, u32x4* __restrict__ wf,
+                                                  u32x4* __restrict__ wg, int* __restrict__ flags) {
+    const long nf = (long)tap_chunks(C) * 9 * 128 * ((K + 63) / 64), ng = wg ? (long)tap_chunks(K) * 9 * 128 * ((C + 63) / 64) : 0;
     const long q = (long)blockIdx.x * NT + threadIdx.x;
-    if (q < nf) {
-        const int r = (int)(q % Kpad);
-        const long ct = q / Kpad;
-        const int t = (int)(ct % 9), c = (int)(ct / 9);
-        wf[q] = r < K ? w[((long)r * C + c) * 9 + t] : 0.f;
-    } else if (q < nf + ng) {
-        const long p = q - nf;
-        const int r = (int)(p % Cpad);
-        const long ct = p / Cpad;
-        const int t = (int)(ct % 9), co = (int)(ct / 9);
-        wg[p] = r < C ? w[((long)co * C + r) * 9 + (8 - t)] : 0.f;
+    u16x2 tiny = {0xffff, 0xffff};
+    if (q < nf + ng) {
+        const bool back = q >= nf;
+        const long e = back ? q - nf : q;
+        const int lane = (int)(e & 63), i = (int)(e >> 6) & 1;
+        const long rest = e >> 7;
+        const int t = (int)(rest % 9);
+        const long rc = rest / 9;
+        const int Cin = back ? K : C, R = back ? C : K, chunks = tap_chunks(Cin);
+        const int ch = (int)(rc % chunks), rt = (int)(rc / chunks);
+        const int r = 64 * rt + 32 * i + (lane & 31), c0 = 16 * ch + 8 * (lane >> 5);
+        float v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int cin = c0 + k;
+            v[k] = (r < R && cin < Cin) ? (back ? w[((long)cin * C + r) * 9 + (8 - t)] : w[((long)r * C + cin) * 9 + t]) : 0.f;
+        }
+        u32x4 c[3];
+        split8(v, c, tiny);
+        u32x4* dst = (back ? wg : wf) + ((rc * 9 + t) * 3 * 2 + i) * 64 + lane;
+#pragma unroll
+        for (int part = 0; part < 3; ++part) dst[part * 128] = c[part];
     }
+    const int any = __syncthreads_or(any_tiny(tiny));
+    if (threadIdx.x == 0) flags[blockIdx.x] = any;
 }
 
 // ------------------------------------------------------------------------------------------
-// tap kernel: o[r][y][x] = sum_{cin, ty, tx} wt[cin][3 ty + tx][r] * src[cin][y + ty + ofs][x + tx + ofs]
+// tap kernel: o[r][y][x] = sum_{cin, ty, tx} w(cin, 3 ty + tx, r) * src[cin][y + ty + ofs][x + tx + ofs]
 //
-// Block: 256 threads, a 64-row (r) x (64 x 4 pixel) output tile.  Wave w owns pixel row
-// y0 + w: 2 x 2 MFMA 32 x 32 tiles (r halves x pixel halves).  Input channels advance CC at a
-// time (CC = 16 with one source, 8 with two); each step stages the (4+2) x (64+2) patch of
-// every channel and the 9 x 64 weight rows in LDS.  The next step's global loads are issued
-// into registers before the MFMAs of the current one.  The MFMA k pair (lane / 32) is a pair
-// of channels at the same tap, so every LDS read has a lane base plus an immediate offset.
+// Block: TY waves, wave w owning pixel row y0 + w of a 64-row (r) x (TX x TY pixel) output tile
+// as 2 x NJ MFMA 32 x 32 tiles (r halves x pixel halves; TX = 32 NJ).  Input channels advance 16
+// at a time: the (TY+2) x (TX+2) patch of the chunk is split into bf16 parts in LDS
+// (split_bf16.hpp), a 16-byte cell per pixel, part and eight channels, so that a tap's pixel
+// fragment is one 128-bit read at a shifted pixel and each element is split once for its 9 taps
+// and 64 rows.  The weight fragments come split from prep_kernel.  A tap is one k step of 16
+// channels, six bf16 products per tile and source-weight pair; its successor's fragments are
+// read while its MFMAs run, and the next chunk is loaded into registers meanwhile.
+// One source (NP = 1; adjoint): NJ = 2, and the weights go through LDS with the patch.  Read
+// from the cache beside the MFMAs instead, a tap's weights wait for every older load of the
+// wave, the next chunk's pixels from HBM among them (loads return in order).  Eight rows give
+// two waves a SIMD.
+// Two sources (NP = 2; tangent, HVP: four products a tap into two outputs): NJ = 1, the weights
+// (two sets, too many for LDS) from the cache.  The two outputs' sums are kept per chunk and then
+// added to their totals, which more than halves their rounding (a tangent's loss sums products
+// of both that cancel).
+// Measured, us with fp32 MFMAs -> split: 8 x 64 -> 64 x 256^2, forward 391 -> 287, xpb 385 -> 270;
+// the matrix cores are busy for 40 % of it.  Without the MFMAs' operands being staged, the
+// MFMAs and the epilogue alone take 186 and 157 us (672 and 406 MB of HBM traffic); weights
+// from the cache with four rows a block: 306 and 290; the splitting interleaved with the MFMAs
+// over a double-buffered patch: no faster.  Error against 64 bits 5.0e-7 -> 4.2e-7 (one source),
+// 3.0e-7 -> 1.8e-7 (two).
+// A block that meets an element which the split cannot hold forms its tile again by
+// v_mfma_f32_32x32x2_f32 with operands straight from memory.
 // ------------------------------------------------------------------------------------------
-constexpr int TX = 64, TY = 4, RT = 64;
-constexpr int PXW = TX + 2, PYH = TY + 2, PPL = PXW * PYH;  // patch row, rows, plane (floats)
-constexpr int KW = 9 * RT;                                    // weight floats per channel
+constexpr int RT = 64, CC = 16;
+constexpr int WCELLS = 9 * 6 * 64;   // weight cells of a chunk and row tile
+enum { FWD_B, FWD_D, FWD_HV, DG_B, DG_HV };
+constexpr int tap_sources(int mode) { return mode == FWD_B || mode == DG_B ? 1 : 2; }
+constexpr int tap_width(int mode) { return tap_sources(mode) == 1 ? 64 : 32; }
 
 struct TapArgs {
-    const float* src[2];  // sources (n, cin, SH, SW)
-    const float* wt[2];   // weights [cin][9][Rpad]
+    const float* src[2];   // sources (n, cin, SH, SW)
+    const u32x4* wt[2];    // split weights (prep_kernel)
+    const float* w[2];     // the weights themselves: (r, cin, t) at w[r * wr + cin * wc + (flip ? 8 - t : t)]
+    long wr, wc;
+    bool flip;
+    const int* flags;      // prep_kernel's, nflags of them
+    int nflags;
     int Cin, R, Rpad, N;
     int SH, SW, ofs;      // source plane and patch origin offset
     int H, W;             // output domain
@@ -95,157 +139,267 @@ struct TapArgs {
     double* partials;     // loss sums per block
 };
 
-template <int MODE>
-__global__ __launch_bounds__(NT, (MODE == FWD_B || MODE == DG_B) ? 2 : 1) void tap_kernel(TapArgs a) {
-    constexpr int NP = (MODE == FWD_B || MODE == DG_B) ? 1 : 2;  // sources = weight sets = outputs
-    constexpr int CC = 16 / NP;
-    constexpr int PSZ = CC * PPL, WSZ = CC * KW;
-    constexpr int WLD = NP * WSZ / 4 / NT;
-    static_assert(NP * WSZ % (4 * NT) == 0, "weight stage");
+template <int MODE, int TY>
+__global__ __launch_bounds__(64 * TY) void tap_kernel(TapArgs a) {
+    constexpr int NP = tap_sources(MODE);  // sources = weight sets = outputs
+    constexpr int TX = tap_width(MODE), NJ = TX / 32;
+    constexpr int NTH = 64 * TY, PXW = TX + 2, PYH = TY + 2, PPL = PXW * PYH;  // patch row, rows, pixels
+    constexpr int PLANE = PPL * 16;                                // bytes of one (part, octet) plane
+    constexpr bool WLDS = NP == 1;                                 // weights staged in LDS
+    constexpr int WPT = WLDS ? (WCELLS + NTH - 1) / NTH : 1;       // weight cells of a thread
     constexpr bool FWD = MODE == FWD_B || MODE == FWD_D || MODE == FWD_HV;
     constexpr int NV = MODE == FWD_B ? 1 : 2;
 
-    __shared__ float lds[NP * (PSZ + WSZ)];
+    __shared__ __attribute__((aligned(16))) char lds[NP * 6 * PLANE];
+    __shared__ u32x4 wlds[WLDS ? WCELLS : 1];
     __shared__ double red[16 * NV];
-    float* Ps = lds;
-    float* Ws = lds + NP * PSZ;
 
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, l32 = lane & 31;
     const int x0 = blockIdx.x * TX, y0 = blockIdx.y * TY;
     const int rtiles = a.Rpad / RT;
     const int n = blockIdx.z / rtiles, rt = blockIdx.z - n * rtiles;
+    const int nchunks = tap_chunks(a.Cin);
 
-    // Patch staging by rows: the NP * CC * PYH = 96 patch rows of PXW = 66 floats; wave w
-    // takes rows w, w + 4, ..., one column per lane (columns 0..63), so the channel, row and
-    // row bounds are wave-uniform (scalar) and a lane's address is a row base plus its lane;
-    // columns 64, 65 of every row go to threads 0..191, one element each.
-    constexpr int PROWS = NP * CC * PYH, RPW = PROWS / 4;
-    static_assert(PROWS % 4 == 0 && PXW == 66 && 2 * PROWS <= NT, "patch rows");
-    float pr[RPW + 1];
-    float4 wr[WLD];
-    // Staging loads are buffer loads: a scalar resource per source image n (and per weight
-    // set), the row part of a patch address as a scalar offset (patch rows are wave-uniform)
-    // and the column as the lane's offset.  An element outside the source reads offset =
-    // the resource's size, which returns 0.  Vector registers hold no 64-bit addresses, so the
-    // staging fits two waves per SIMD without spilling.  (The host keeps one image of a
-    // source and a weight set under 2^31 bytes.)
+    // Patch staging: a cell is one pixel's eight channels of an octet; a source's 2 x PYH x PXW
+    // cells (octet, row, column) are shared out over the threads in order, so that consecutive
+    // lanes load consecutive pixels.  The loads are buffer loads: a scalar resource per source
+    // image n, the channel as a scalar offset, the rest as the lane's.  An element outside the
+    // source reads an offset past the resource, which returns 0.  (The host keeps one image of
+    // a source under 2^31 bytes.)
+    constexpr int NCELL = (2 * PPL + NTH - 1) / NTH;
+    float pr[NP][NCELL][8];
+    u32x4 wr[WPT];
     const long plane = (long)a.SH * a.SW;
     const uint32_t sbytes = (uint32_t)((long)a.Cin * plane * 4);
-    const uint32_t wbytes = (uint32_t)((long)a.Cin * 9 * a.Rpad * 4);
-    __amdgpu_buffer_rsrc_t rs[NP], rw[NP];
+    constexpr uint32_t kPast = 0x80000000u;
+    __amdgpu_buffer_rsrc_t rs[NP];
 #pragma unroll
-    for (int p = 0; p < NP; ++p) {
+    for (int p = 0; p < NP; ++p)
         rs[p] = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.src[p] + (long)n * a.Cin * plane), (short)0, sbytes,
                                                   kBufWord3);
-        rw[p] = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.wt[p] + rt * RT), (short)0, wbytes, kBufWord3);
+    uint32_t voff[NCELL];  // the cell's byte offset at channel 8 octet
+    int clim[NCELL];       // channels from there on
+    int coff[NCELL];       // the cell's place in LDS (part 0)
+#pragma unroll
+    for (int k = 0; k < NCELL; ++k) {
+        const int e = threadIdx.x + NTH * k, row = e / PXW, col = e - row * PXW;
+        const int oct = row >= PYH, ty = row - oct * PYH;
+        const int sy = y0 + ty + a.ofs, sx = x0 + col + a.ofs;
+        const bool in = e < 2 * PPL && (unsigned)sy < (unsigned)a.SH && (unsigned)sx < (unsigned)a.SW;
+        clim[k] = in ? a.Cin - 8 * oct : 0;
+        voff[k] = in ? (uint32_t)((8 * oct * plane + (long)sy * a.SW + sx) * 4) : kPast;
+        coff[k] = oct * PLANE + (ty * PXW + col) * 16;
     }
-    const int sx_l = x0 + lane + a.ofs;
-    const uint32_t lane_col = (unsigned)sx_l < (unsigned)a.SW ? (uint32_t)sx_l * 4u : sbytes;
-    auto load = [&](int c0) {
+    auto load = [&](int ch) {
+        if constexpr (WLDS) {
+            const u32x4* w = a.wt[0] + ((long)rt * nchunks + ch) * WCELLS;
 #pragma unroll
-        for (int i = 0; i < RPW; ++i) {
-            const int rr = wave + 4 * i;  // wave-uniform patch row (p, cc, ty)
-            const int p = NP == 1 ? 0 : rr / (CC * PYH);
-            const int rem = rr - p * (CC * PYH);
-            const int cc = rem / PYH, ty = rem - cc * PYH;
-            const int c = c0 + cc, sy = y0 + ty + a.ofs;
-            const bool ok = c < a.Cin && (unsigned)sy < (unsigned)a.SH;
-            const uint32_t soff = ok ? (uint32_t)(((long)c * a.SH + sy) * a.SW * 4) : 0u;
-            const uint32_t voff = ok ? lane_col : sbytes;
-            pr[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(p ? rs[NP - 1] : rs[0], voff, soff, 0));
+            for (int q = 0; q < WPT; ++q)
+                if (WCELLS % NTH == 0 || threadIdx.x + NTH * q < WCELLS) wr[q] = w[threadIdx.x + NTH * q];
         }
-        if (threadIdx.x < 2 * PROWS) {
-            // columns 64, 65: the row varies across a wave, so the whole offset is the lane's
-            const int rr = threadIdx.x >> 1, col = 64 + (threadIdx.x & 1);
-            const int p = NP == 1 ? 0 : rr / (CC * PYH);
-            const int rem = rr - p * (CC * PYH);
-            const int cc = rem / PYH, ty = rem - cc * PYH;
-            const int c = c0 + cc, sy = y0 + ty + a.ofs, sx = x0 + col + a.ofs;
-            float v = 0.f;
-            if (c < a.Cin && (unsigned)sy < (unsigned)a.SH && (unsigned)sx < (unsigned)a.SW)
-                v = a.src[p][((long)(n * a.Cin + c) * a.SH + sy) * a.SW + sx];
-            pr[RPW] = v;
-        }
-        const uint32_t wsoff = (uint32_t)((long)c0 * 9 * a.Rpad * 4);
 #pragma unroll
-        for (int q = 0; q < WLD; ++q) {
-            const int f = threadIdx.x + q * NT;  // float4 slot of [w][cc][t][r]
-            const int wi = NP == 1 ? 0 : __builtin_amdgcn_readfirstlane(f / (WSZ / 4));  // uniform per wave
-            const int rem = f - wi * (WSZ / 4);
-            const int row = rem / (RT / 4), r4 = (rem - row * (RT / 4)) * 4;
-            const int cc = row / 9, t = row - cc * 9;
-            const uint32_t voff = c0 + cc < a.Cin ? (uint32_t)(((cc * 9 + t) * a.Rpad + r4) * 4) : wbytes;
-            const v4f x = __builtin_amdgcn_raw_buffer_load_b128(wi ? rw[NP - 1] : rw[0], voff, wsoff, 0);
-            wr[q] = make_float4(x.x, x.y, x.z, x.w);
-        }
+        for (int k = 0; k < NCELL; ++k)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int c = CC * ch + e;
+                const uint32_t soff = (uint32_t)(min(c, a.Cin) * plane * 4), v = c < clim[k] ? voff[k] : kPast;
+#pragma unroll
+                for (int p = 0; p < NP; ++p)
+                    pr[p][k][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs[p], v, soff, 0));
+            }
     };
+    u16x2 tiny = {0xffff, 0xffff};
     auto store = [&]() {
-        // patch row rr = (p, cc, ty) is at Ps + p * PSZ + cc * PPL + ty * PXW = Ps + rr * PXW
 #pragma unroll
-        for (int i = 0; i < RPW; ++i) Ps[(wave + 4 * i) * PXW + lane] = pr[i];
-        if (threadIdx.x < 2 * PROWS) Ps[(threadIdx.x >> 1) * PXW + 64 + (threadIdx.x & 1)] = pr[RPW];
+        for (int p = 0; p < NP; ++p)
 #pragma unroll
-        for (int q = 0; q < WLD; ++q) {
-            const int f = threadIdx.x + q * NT;
-            *reinterpret_cast<float4*>(Ws + 4 * f) = wr[q];
+            for (int k = 0; k < NCELL; ++k) {
+                u32x4 c[3];
+                split8(pr[p][k], c, tiny);
+                if ((2 * PPL) % NTH == 0 || threadIdx.x + NTH * k < 2 * PPL)
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x4*>(lds + (p * 6 + 2 * q) * PLANE + coff[k]) = c[q];
+            }
+        if constexpr (WLDS) {
+#pragma unroll
+            for (int q = 0; q < WPT; ++q)
+                if (WCELLS % NTH == 0 || threadIdx.x + NTH * q < WCELLS) wlds[threadIdx.x + NTH * q] = wr[q];
         }
     };
 
-    floatx16 acc[NP][2][2];
+    floatx16 acc[NP][2][NJ];
+    auto clear = [&]() {
 #pragma unroll
-    for (int o = 0; o < NP; ++o)
+        for (int o = 0; o < NP; ++o)
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+                for (int j = 0; j < NJ; ++j)
 #pragma unroll
-                for (int q = 0; q < 16; ++q) acc[o][i][j][q] = 0.f;
+                    for (int q = 0; q < 16; ++q) acc[o][i][j][q] = 0.f;
+    };
+    clear();
 
-    // lane bases: patch channel (2 qq + h), row (wave + ky), column (32 j + l32 + kx);
-    // weight row (2 qq + h, t), column 32 i + l32
-    const int pbase = h * PPL + wave * PXW + l32;
-    const int wbase = h * KW + l32;
-    const int nchunks = (a.Cin + CC - 1) / CC;
-    if (nchunks > 0) load(0);
+    // fragments, two sets: a tap's are read during the tap before
+    bf16x8 wv[2][NP][2][3], pv[2][NP][NJ][3];
+    auto read_weights = [&](int ch, int t, int buf) {
+        if constexpr (WLDS) {
+#pragma unroll
+            for (int q = 2; q >= 0; --q)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    wv[buf][0][i][q] = __builtin_bit_cast(bf16x8, wlds[(t * 6 + q * 2 + i) * 64 + lane]);
+            return;
+        }
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<u32x4*>(a.wt[p] + ((long)rt * nchunks + ch) * (9 * 6 * 64)), (short)0, 9 * 6 * 1024, kBufWord3);
+#pragma unroll
+            for (int q = 2; q >= 0; --q)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    wv[buf][p][i][q] = __builtin_bit_cast(
+                        bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rw, (uint32_t)lane * 16u, (uint32_t)(t * 6 + q * 2 + i) * 1024u, 0));
+        }
+    };
+    auto read_pixels = [&](int t, int buf) {
+        const int ky = t / 3, kx = t % 3;
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+                    pv[buf][p][j][q] = *reinterpret_cast<const bf16x8*>(lds + (p * 6 + 2 * q + h) * PLANE + ((wave + ky) * PXW + kx + 32 * j + l32) * 16);
+    };
+    // two sources: the chunks' sums (acc) are added up here
+    floatx16 tot[NP == 2 ? NP : 1][2][NJ];
+    if constexpr (NP == 2) {
+#pragma unroll
+        for (int o = 0; o < NP; ++o)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) tot[o][i][j] = acc[o][i][j];
+    }
+    if (nchunks > 0) {
+        load(0);
+        if (!WLDS) read_weights(0, 0, 0);
+    }
     for (int ch = 0; ch < nchunks; ++ch) {
         __syncthreads();
         store();
         __syncthreads();
-        if (ch + 1 < nchunks) load((ch + 1) * CC);
-        // k steps st = (channel pair qq, tap t); the fragments of step st+1 are read from LDS
-        // while the MFMAs of step st run (two register sets; the scheduling barriers keep
-        // the compiler from sinking each read to its use)
-        constexpr int NSTEP = CC / 2 * 9;
-        float pf[2][NP][2], wf[2][NP][2];
-        auto frag = [&](int st, int buf) {
-            const int qq = st / 9, t = st % 9, ky = t / 3, kx = t % 3;
-#pragma unroll
-            for (int p = 0; p < NP; ++p)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) pf[buf][p][j] = Ps[p * PSZ + pbase + 2 * qq * PPL + ky * PXW + kx + 32 * j];
-#pragma unroll
-            for (int p = 0; p < NP; ++p)
-#pragma unroll
-                for (int i = 0; i < 2; ++i) wf[buf][p][i] = Ws[p * WSZ + wbase + (2 * qq * 9 + t) * RT + 32 * i];
-        };
-        frag(0, 0);
-#pragma unroll
-        for (int st = 0; st < NSTEP; ++st) {
-            const int b = st & 1;
-            if (st + 1 < NSTEP) frag(st + 1, b ^ 1);
+        if (ch + 1 < nchunks) load(ch + 1);
+        if (WLDS) read_weights(ch, 0, 0);
+        read_pixels(0, 0);
+        auto tap = [&](int t, int b) {
+            if (t < 8) {
+                read_pixels(t + 1, b ^ 1);
+                read_weights(ch, t + 1, b ^ 1);
+            } else if (!WLDS && ch + 1 < nchunks) {
+                read_weights(ch + 1, 0, b ^ 1);
+            }
             __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int x = 0; x < 6; ++x)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j) {
+                        acc[0][i][j] = mfma_bf16(wv[b][0][i][kSplitB[x]], pv[b][0][j][kSplitA[x]], acc[0][i][j]);
+                        if constexpr (NP == 2) {
+                            acc[1][i][j] = mfma_bf16(wv[b][1][i][kSplitB[x]], pv[b][0][j][kSplitA[x]], acc[1][i][j]);
+                            acc[1][i][j] = mfma_bf16(wv[b][0][i][kSplitB[x]], pv[b][1][j][kSplitA[x]], acc[1][i][j]);
+                        }
+                    }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+            tap(t, t & 1);
+            if constexpr (NP == 2) {
+                if (t != 8) continue;
+#pragma unroll
+                for (int o = 0; o < NP; ++o)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                            for (int q = 0; q < 16; ++q) {
+                                tot[o][i][j][q] += acc[o][i][j][q];
+                                acc[o][i][j][q] = 0.f;
+                            }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if constexpr (!WLDS) {
+            // (nine taps leave the next chunk's first weights in the other set: it is copied over)
+#pragma unroll
+            for (int p = 0; p < NP; ++p)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) wv[0][p][i][q] = wv[1][p][i][q];
+        }
+    }
+
+    if constexpr (NP == 2) {
+#pragma unroll
+        for (int o = 0; o < NP; ++o)
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    acc[0][i][j] = mfma(wf[b][0][i], pf[b][0][j], acc[0][i][j]);
-                    if constexpr (NP == 2) {
-                        acc[1][i][j] = mfma(wf[b][1][i], pf[b][0][j], acc[1][i][j]);
-                        acc[1][i][j] = mfma(wf[b][0][i], pf[b][1][j], acc[1][i][j]);
+                for (int j = 0; j < NJ; ++j) acc[o][i][j] = tot[o][i][j];
+    }
+    // an element that the split cannot hold, or a sum that is not finite: the tile again in fp32
+    {
+        float z = 0.f;
+#pragma unroll
+        for (int o = 0; o < NP; ++o)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) z = __builtin_fmaf(acc[o][i][j][q], 0.f, z);
+        bool redo = z != 0.f || any_tiny(tiny);
+        for (int k = threadIdx.x; k < a.nflags; k += NTH) redo = redo || a.flags[k];
+        if (__syncthreads_or(redo)) {
+            clear();
+            for (int c0 = 0; c0 < a.Cin; c0 += 2)
+                for (int t = 0; t < 9; ++t) {
+                    const int c = c0 + h, ky = t / 3, kx = t - 3 * ky;
+                    const int sy = y0 + wave + ky + a.ofs;
+                    float wf[NP][2], pf[NP][NJ];
+#pragma unroll
+                    for (int p = 0; p < NP; ++p) {
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) {
+                            const int r = rt * RT + 32 * i + l32;
+                            wf[p][i] = c < a.Cin && r < a.R ? a.w[p][r * a.wr + c * a.wc + (a.flip ? 8 - t : t)] : 0.f;
+                        }
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j) {
+                            const int sx = x0 + 32 * j + l32 + kx + a.ofs;
+                            pf[p][j] = c < a.Cin && (unsigned)sy < (unsigned)a.SH && (unsigned)sx < (unsigned)a.SW
+                                           ? a.src[p][((long)(n * a.Cin + c) * a.SH + sy) * a.SW + sx] : 0.f;
+                        }
                     }
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j) {
+                            acc[0][i][j] = mfma(wf[0][i], pf[0][j], acc[0][i][j]);
+                            if constexpr (NP == 2) {
+                                acc[1][i][j] = mfma(wf[1][i], pf[0][j], acc[1][i][j]);
+                                acc[1][i][j] = mfma(wf[0][i], pf[1][j], acc[1][i][j]);
+                            }
+                        }
                 }
-            __builtin_amdgcn_sched_barrier(0);
         }
     }
 
@@ -263,7 +417,7 @@ __global__ __launch_bounds__(NT, (MODE == FWD_B || MODE == DG_B) ? 2 : 1) void t
     // compiler knows, so interleaving would serialise one HBM round trip per element.
     constexpr bool RMW = MODE != FWD_D;
     constexpr int NR = (MODE == FWD_HV || MODE == DG_HV) ? 2 : 1;
-    float pre[NR][2][2][16];
+    float pre[NR][2][NJ][16];
     auto index = [&](int i, int j, int q, long& oi) {
         const int x = x0 + 32 * j + l32;
         const int r = rt * RT + 32 * i + 8 * (q >> 2) + 4 * h + (q & 3);
@@ -276,7 +430,7 @@ __global__ __launch_bounds__(NT, (MODE == FWD_B || MODE == DG_B) ? 2 : 1) void t
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int j = 0; j < NJ; ++j)
 #pragma unroll
                 for (int q = 0; q < 16; ++q) {
                     long oi;
@@ -288,7 +442,7 @@ __global__ __launch_bounds__(NT, (MODE == FWD_B || MODE == DG_B) ? 2 : 1) void t
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int q = 0; q < 16; ++q) {
                 long oi;
@@ -676,7 +830,7 @@ int32_t check(int64_t N, int64_t C, int64_t K, int64_t H, int64_t W, const char*
     d.Hp = d.H + 2; d.Wp = d.W + 2;
     d.Kpad = (d.K + 63) / 64 * 64;
     d.Cpad = (d.C + 63) / 64 * 64;
-    const long tapblocks = (long)((d.W + TX - 1) / TX) * ((d.H + TY - 1) / TY) * d.N * (d.Kpad / 64);
+    const long tapblocks = (long)((d.W + 63) / 64) * ((d.H + 3) / 4) * d.N * (d.Kpad / 64);
     if (tapblocks * 2 > kPartialSlots) return set_error(STADE_HIP_ERANGE, "%s: sizes out of range", fn);
     return STADE_HIP_OK;
 }
@@ -685,9 +839,21 @@ inline size_t up64(size_t n) { return (n + 63) / 64 * 64; }
 
 template <int MODE>
 hipError_t launch_tap(const TapArgs& a, const char* name, hipStream_t stream, unsigned& nblocks) {
-    dim3 grid((a.W + TX - 1) / TX, (a.H + TY - 1) / TY, a.N * (a.Rpad / RT));
+    // one source: eight pixel rows a block where that still gives every CU one (two waves a
+    // SIMD; the halo rows are a quarter of the patch instead of a half), otherwise four
+    constexpr int TX = tap_width(MODE);
+    const long tiles = (long)((a.W + TX - 1) / TX) * a.N * (a.Rpad / RT);
+    const bool tall = tap_sources(MODE) == 1 && tiles * ((a.H + 7) / 8) >= gemm::device_cus();
+    const int ty = tall ? 8 : 4;
+    dim3 grid((a.W + TX - 1) / TX, (a.H + ty - 1) / ty, a.N * (a.Rpad / RT));
     nblocks = grid.x * grid.y * grid.z;
-    STADE_TIMED(name, stream, (tap_kernel<MODE><<<grid, NT, 0, stream>>>(a)));
+    if constexpr (tap_sources(MODE) == 1) {
+        if (tall) {
+            STADE_TIMED(name, stream, (tap_kernel<MODE, 8><<<grid, 512, 0, stream>>>(a)));
+            return hipGetLastError();
+        }
+    }
+    STADE_TIMED(name, stream, (tap_kernel<MODE, 4><<<grid, 256, 0, stream>>>(a)));
     return hipGetLastError();
 }
 
@@ -719,15 +885,22 @@ int32_t run(const Ptrs& p, const Dims& d, hipStream_t stream) {
     WsCall call_(stream);
     Workspace* ws = call_.ws;
     if (!ws) return STADE_HIP_ENOMEM;
-    const size_t nwf = up64((size_t)d.C * 9 * d.Kpad), nwg = up64((size_t)d.K * 9 * d.Cpad);
+    // split weights: 16-byte cells, 3 parts of 128 a tap, chunk and row tile (in floats below)
+    const size_t cf = (size_t)tap_chunks(d.C) * 9 * 128 * (d.Kpad / 64), cg = (size_t)tap_chunks(d.K) * 9 * 128 * (d.Cpad / 64);
+    const size_t nwf = cf * 12, nwg = cg * 12;
+    const int nprep = (int)((cf + (MODE == TAN ? 0 : cg) + NT - 1) / NT);
+    const int two = MODE == ADJ ? 1 : 2;
+    const size_t nflag = up64((size_t)two * nprep);
     const size_t nout = up64((size_t)d.N * d.K * d.H * d.W);
     const int ctn = d.Cpad / 64, ktn = d.Kpad / 64;
     const long ntiles = (long)((d.W + WTX - 1) / WTX) * ((d.H + WTY - 1) / WTY) * d.N;
     // ctn is 0 when C = 0 (no weight gradient to form)
     const int nsplit = ctn == 0 ? 0 : (int)std::max(1L, std::min(ntiles, (long)std::max(1, 256 / (ctn * ktn))));
     const size_t npart = (MODE == TAN || d.C == 0) ? 0 : (size_t)nsplit * ctn * ktn * 9 * 4096;
-    const int two = MODE == ADJ ? 1 : 2;
-    const size_t total = two * nwf + (MODE == TAN ? 0 : two * nwg + two * nout) + npart;
+    // the loss partials of the forward pass, where they do not fit the workspace's own
+    const size_t nloss = 2 * (size_t)((d.W + tap_width(FWD_D) - 1) / tap_width(FWD_D)) * ((d.H + 3) / 4) * d.N * (d.Kpad / 64);
+    const bool own_loss = MODE != ADJ && nloss > (size_t)kPartialSlots;
+    const size_t total = two * nwf + (MODE == TAN ? 0 : two * nwg + two * nout) + nflag + up64(npart) + (own_loss ? 2 * nloss : 0);
     float* base = (float*)scratch(sizeof(float) * total + 256);
     if (!base) return scratch_error();
     float* wf0 = base;
@@ -736,28 +909,24 @@ int32_t run(const Ptrs& p, const Dims& d, hipStream_t stream) {
     float* wg1 = wg0 + nwg;
     float* G = wg0 + (MODE == TAN ? 0 : two * nwg);
     float* GD = G + nout;
-    float* part = G + (MODE == TAN ? 0 : two * nout);
+    int* flags = (int*)(G + (MODE == TAN ? 0 : two * nout));
+    float* part = (float*)(flags + nflag);
+    double* const lpart = own_loss ? (double*)(part + up64(npart)) : ws->partials;
 
-    // weights in tap-kernel layouts
-    {
-        const long n = (long)d.C * 9 * d.Kpad + (MODE == TAN ? 0 : (long)d.K * 9 * d.Cpad);
-        const unsigned nb = (unsigned)((n + NT - 1) / NT);
-        if (n > 0) {
-            STADE_TIMED("conv_prep", stream, (prep_kernel<<<nb, NT, 0, stream>>>(p.w, d.C, d.K, wf0, d.Kpad,
-                                                                                 MODE == TAN ? nullptr : wg0, d.Cpad)));
-            STADE_LAUNCHED("conv3x3 prep_kernel");
-            if (MODE != ADJ) {
-                STADE_TIMED("conv_prep", stream, (prep_kernel<<<nb, NT, 0, stream>>>(p.wd, d.C, d.K, wf1, d.Kpad,
-                                                                                     MODE == TAN ? nullptr : wg1, d.Cpad)));
-                STADE_LAUNCHED("conv3x3 prep_kernel");
-            }
-        }
+    // weights in the tap kernel's form
+    for (int s = 0; s < two && nprep > 0; ++s) {
+        STADE_TIMED("conv_prep", stream, (prep_kernel<<<nprep, NT, 0, stream>>>(s ? p.wd : p.w, d.C, d.K, (u32x4*)(s ? wf1 : wf0),
+                                                                               MODE == TAN ? nullptr : (u32x4*)(s ? wg1 : wg0),
+                                                                               flags + s * nprep)));
+        STADE_LAUNCHED("conv3x3 prep_kernel");
     }
     // forward: out (and outd), loss (and lossd); adjoint seeds g (and gd), outb (and outbd) reset
     {
         TapArgs a{};
         a.src[0] = p.xp; a.src[1] = p.xpd;
-        a.wt[0] = wf0; a.wt[1] = wf1;
+        a.wt[0] = (u32x4*)wf0; a.wt[1] = (u32x4*)wf1;
+        a.w[0] = p.w; a.w[1] = p.wd; a.wr = 9L * d.C; a.wc = 9; a.flip = false;
+        a.flags = flags; a.nflags = two * nprep;
         a.Cin = d.C; a.R = d.K; a.Rpad = d.Kpad; a.N = d.N;
         a.SH = d.Hp; a.SW = d.Wp; a.ofs = 0;
         a.H = d.H; a.W = d.W;
@@ -765,7 +934,7 @@ int32_t run(const Ptrs& p, const Dims& d, hipStream_t stream) {
         a.OH = d.H; a.OW = d.W; a.oofs = 0;
         a.g0 = G; a.g1 = GD; a.ob = p.outb; a.obd = p.outbd;
         a.lossb = p.lossb; a.lossbd = p.lossbd;
-        a.partials = ws->partials;
+        a.partials = lpart;
         unsigned nblocks = 0;
         hipError_t e;
         if (MODE == ADJ) e = launch_tap<FWD_B>(a, "conv_fwd", stream, nblocks);
@@ -773,9 +942,9 @@ int32_t run(const Ptrs& p, const Dims& d, hipStream_t stream) {
         else e = launch_tap<FWD_HV>(a, "conv_fwd_hv", stream, nblocks);
         if (e != hipSuccess) return check_hip(e, "conv3x3 tap_kernel (forward)");
         if (MODE == ADJ) {
-            STADE_TIMED("conv_loss", stream, (loss_kernel<1><<<1, NT, 0, stream>>>(ws->partials, (int)nblocks, p.loss, nullptr)));
+            STADE_TIMED("conv_loss", stream, (loss_kernel<1><<<1, NT, 0, stream>>>(lpart, (int)nblocks, p.loss, nullptr)));
         } else {
-            STADE_TIMED("conv_loss", stream, (loss_kernel<2><<<1, NT, 0, stream>>>(ws->partials, (int)nblocks, p.loss, p.lossd)));
+            STADE_TIMED("conv_loss", stream, (loss_kernel<2><<<1, NT, 0, stream>>>(lpart, (int)nblocks, p.loss, p.lossd)));
         }
         STADE_LAUNCHED("conv3x3 loss_kernel");
     }
@@ -793,7 +962,9 @@ int32_t run(const Ptrs& p, const Dims& d, hipStream_t stream) {
     {
         TapArgs a{};
         a.src[0] = G; a.src[1] = GD;
-        a.wt[0] = wg0; a.wt[1] = wg1;
+        a.wt[0] = (u32x4*)wg0; a.wt[1] = (u32x4*)wg1;
+        a.w[0] = p.w; a.w[1] = p.wd; a.wr = 9; a.wc = 9L * d.C; a.flip = true;
+        a.flags = flags; a.nflags = two * nprep;
         a.Cin = d.K; a.R = d.C; a.Rpad = d.Cpad; a.N = d.N;
         a.SH = d.H; a.SW = d.W; a.ofs = -1;
         a.H = d.H; a.W = d.W;

@@ -12,12 +12,8 @@
 // W1d * X + W1 * Xd is one launch.  A dual launch instead reads both segments in the same K
 // steps and writes two outputs, P = A0 B0 and Q = A0 B1 + A1 B0 (a product with its tangent).
 //
-// Arithmetic: split bf16.  Each operand element is written as h + m + l, three bf16 values
-// that hold its 24 bits exactly (h = bf16(a), m = bf16(a - h), l = a - h - m; both
-// subtractions are exact), and a product is the sum of six bf16 matrix products accumulated
-// in fp32, small ones first: l h + h l + m m + m h + h m + h h.  The three dropped products
-// are at most 2^-24 of h h together and the bf16 products themselves are exact, so what is
-// left is the rounding of the fp32 accumulation, once per instruction and 16 k, where
+// Arithmetic: six bf16 products of operands split into three bf16 parts (split_bf16.hpp).  What
+// is left is the rounding of the fp32 accumulation, once per instruction and 16 k, where
 // v_mfma_f32_32x32x2_f32 rounds every 2 k: against 64 bits (N(0, 1) times U(0, 1) operands) the
 // normwise error is 4.0e-7 at K = 784 and 9.9e-7 at K = 4096, of v_mfma_f32_32x32x2_f32 5.0e-7
 // and 1.1e-6.  The matrix cores run bf16 at 16 times the fp32 rate, so six products leave a
@@ -26,17 +22,15 @@
 // loop now is the splitting (12 vector instructions a pair of elements, 104 a wave and step
 // beside 24 MFMAs) and the LDS traffic that a block's two waves a SIMD do not hide wholly:
 // without the splitting the same loop runs at 270 TFLOP/s, with it at 180.
-// An element whose l part would not be exact (0 < |a| < 2^-110, below bf16's smallest
-// subnormal) and an element that is not finite or rounds to infinity (which leaves the tile
-// with a non-finite sum) are noticed by the block, which then forms its tile again with
-// fp32 matrix instructions (fp32_loop): the results there are those of plain fp32.
+// A block that meets an element the split cannot hold forms its tile again with fp32 matrix
+// instructions (fp32_loop): the results there are those of plain fp32.
 //
 // Tiling: a 256-thread block (4 waves) computes a 128 x BNT tile of C (BNT = 128 or 64);
 // each wave a 64 x BNT/2 part as 2 x BNT/64 MFMA 32 x 32 tiles.  K advances 16 at a time
 // through two LDS buffers: while a step's MFMAs run from one, the next step is split and stored to
 // the other and the step after that is being loaded; one barrier a step, and two blocks a CU,
-// so that one block's splitting overlaps the other's MFMAs.  The partial K steps (K % 16, one a segment) come
-// first, in the prologue, so that the steps of the loop load without tests.
+// so that one block's splitting overlaps the other's MFMAs.  The partial K steps (K % 16, one a
+// segment) come first, in the prologue, so that the steps of the loop load without tests.
 // The MFMA operands are swapped (B tile as the matrix-core A operand) so that the
 // accumulator's lane index runs along m: each epilogue store of a wave covers 32 consecutive
 // rows of a column-major C, a 128-byte segment.
@@ -55,15 +49,10 @@
 #include <type_traits>
 #include <utility>
 
+#include "split_bf16.hpp"
+
 namespace stade {
 namespace gemm {
-
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int BM = 128, KT = 16, NT = 256;
 constexpr int KQ = KT / 4;  // k-planes per step of the fp32 loop
@@ -213,37 +202,6 @@ constexpr int plane_bytes() {
 template <int ROWS>
 constexpr int tile_bytes() {
     return 6 * plane_bytes<ROWS>();
-}
-
-__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
-    uint32_t r;  // (one instruction; from two scalar conversions the compiler makes three)
-    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-__device__ __forceinline__ float bf16_lo(uint32_t v) { return __builtin_bit_cast(float, v << 16); }
-__device__ __forceinline__ float bf16_hi(uint32_t v) { return __builtin_bit_cast(float, v & 0xffff0000u); }
-
-// the smallest 2 |h| - 1 (as bits, so zero counts as the largest) of the elements seen: below
-// kTinyBits an element is nonzero and under 2^-109, where its l part may not be exact
-constexpr unsigned short kTinyBits = ((127 - 109) << 8) - 1;
-
-__device__ __forceinline__ u16x2 twice_less_one(uint32_t h) {
-    u16x2 r;
-    asm("v_pk_mad_u16 %0, %1, 2, -1 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h));
-    return r;
-}
-
-__device__ __forceinline__ void split8(const float (&v)[8], u32x4 (&c)[3], u16x2& tiny) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const uint32_t h = pack_bf16(v[2 * q], v[2 * q + 1]);
-        const float r0 = v[2 * q] - bf16_lo(h), r1 = v[2 * q + 1] - bf16_hi(h);
-        const uint32_t m = pack_bf16(r0, r1);
-        c[0][q] = h;
-        c[1][q] = m;
-        c[2][q] = pack_bf16(r0 - bf16_lo(m), r1 - bf16_hi(m));
-        tiny = __builtin_elementwise_min(tiny, twice_less_one(h));
-    }
 }
 
 // this thread's cell of a ROWS x 16 tile (ROWS = 64: threads 0..127, or, of two such tiles,
@@ -401,22 +359,24 @@ __device__ __forceinline__ void gemm_block(const Args& g, const Epi& epi, int bx
     const int m0 = bx * BM, n0 = by * BNT;
     const int wm = (wave & 1) * 64, wn = (wave >> 1) * (BNT / 2);
 
-    // Both segments' operands in registers (indexing g.seg[s] with a runtime s would reload
-    // them from the kernel-argument segment at every step).
-    const bool two = g.nseg > 1;
-    const long lda0 = g.seg[0].lda, ldb0 = g.seg[0].ldb;
-    const long lda1 = two ? g.seg[1].lda : lda0, ldb1 = two ? g.seg[1].ldb : ldb0;
-    const __amdgpu_buffer_rsrc_t rA0 = operand_rsrc(g.seg[0].A, g.abytes[0]), rA1 = operand_rsrc(g.seg[two].A, g.abytes[two]);
-    const __amdgpu_buffer_rsrc_t rB0 = operand_rsrc(g.seg[0].B, g.bbytes[0]), rB1 = operand_rsrc(g.seg[two].B, g.bbytes[two]);
-    const uint32_t oA0 = cell_offset<A_KM, BM>(lda0, m0, g.M), oA1 = cell_offset<A_KM, BM>(lda1, m0, g.M);
-    const uint32_t oB0 = cell_offset<B_KM, BNT>(ldb0, n0, g.N), oB1 = cell_offset<B_KM, BNT>(ldb1, n0, g.N);
-
     // the K steps of all segments (DUAL: of the shared K), partial ones first; this block's slice
+    const bool two = g.nseg > 1;
     const int total = step_count<DUAL>(g);
     const int t_begin = (int)((long)total * bz / g.ksplit);
     const int t_end = (int)((long)total * (bz + 1) / g.ksplit);
     const int npart = (g.seg[0].K % KT != 0) + (!DUAL && two && g.seg[1].K % KT != 0);
     const int full0 = g.seg[0].K / KT;
+    // Both segments' operands in registers (indexing g.seg[s] with a runtime s would reload
+    // them from the kernel-argument segment at every step).  A slice without a whole step (a
+    // short K) loads none: its whole-step loads all fall past the buffers and return zero.
+    const bool whole = t_end > npart;
+    const long lda0 = whole ? g.seg[0].lda : 0, ldb0 = whole ? g.seg[0].ldb : 0;
+    const long lda1 = whole && two ? g.seg[1].lda : lda0, ldb1 = whole && two ? g.seg[1].ldb : ldb0;
+    const __amdgpu_buffer_rsrc_t rA0 = operand_rsrc(g.seg[0].A, g.abytes[0]), rA1 = operand_rsrc(g.seg[two].A, g.abytes[two]);
+    const __amdgpu_buffer_rsrc_t rB0 = operand_rsrc(g.seg[0].B, g.bbytes[0]), rB1 = operand_rsrc(g.seg[two].B, g.bbytes[two]);
+    const int ma = whole ? g.M : 0, nb = whole ? g.N : 0;
+    const uint32_t oA0 = cell_offset<A_KM, BM>(lda0, m0, ma), oA1 = cell_offset<A_KM, BM>(lda1, m0, ma);
+    const uint32_t oB0 = cell_offset<B_KM, BNT>(ldb0, n0, nb), oB1 = cell_offset<B_KM, BNT>(ldb1, n0, nb);
 
     floatx16 acc[NOP][2][NJ];  // DUAL: [0] P, [1] Q
 #pragma unroll
@@ -445,8 +405,7 @@ __device__ __forceinline__ void gemm_block(const Args& g, const Epi& epi, int bx
     float va[NOP][8], vb[8];
     // a whole step t >= npart
     auto load = [&](int t) {
-        if (t_end <= npart) return;  // the slice has no whole step (a short K)
-        const int u = min(t, t_end - 1) - npart;
+        const int u = max(min(t, t_end - 1) - npart, 0);
         if constexpr (DUAL) {
             const uint32_t sa = (uint32_t)((A_KM ? (long)u * KT : (long)u * KT * lda0) * 4);
             load_cell<A_KM>(va[0], rA0, oA0, sa, (uint32_t)(lda0 * 4));
@@ -514,7 +473,6 @@ __device__ __forceinline__ void gemm_block(const Args& g, const Epi& epi, int bx
     const bool li = m0 + wm + 32 < g.M, lj = n0 + wn + 32 < g.N, l0 = m0 + wm < g.M && n0 + wn < g.N;
     auto mma = [&](auto whole_tag) {
         constexpr bool WHOLE = decltype(whole_tag)::value;
-        constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
         if (!WHOLE && !l0) return;
 #pragma unroll
         for (int x = 0; x < 6; ++x)
@@ -523,10 +481,10 @@ __device__ __forceinline__ void gemm_block(const Args& g, const Epi& epi, int bx
 #pragma unroll
                 for (int j = 0; j < NJ; ++j) {
                     if (!WHOLE && ((i && !li) || (j && !lj))) continue;
-                    acc[0][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[0][j][pb[x]], fa[0][i][pa[x]], acc[0][i][j], 0, 0, 0);
+                    acc[0][i][j] = mfma_bf16(fb[0][j][kSplitB[x]], fa[0][i][kSplitA[x]], acc[0][i][j]);
                     if constexpr (DUAL) {
-                        acc[1][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[1][j][pb[x]], fa[0][i][pa[x]], acc[1][i][j], 0, 0, 0);
-                        acc[1][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[0][j][pb[x]], fa[1][i][pa[x]], acc[1][i][j], 0, 0, 0);
+                        acc[1][i][j] = mfma_bf16(fb[1][j][kSplitB[x]], fa[0][i][kSplitA[x]], acc[1][i][j]);
+                        acc[1][i][j] = mfma_bf16(fb[0][j][kSplitB[x]], fa[1][i][kSplitA[x]], acc[1][i][j]);
                     }
                 }
     };
@@ -564,7 +522,7 @@ __device__ __forceinline__ void gemm_block(const Args& g, const Epi& epi, int bx
                 for (int j = 0; j < NJ; ++j)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) z = __builtin_fmaf(acc[o][i][j][r], 0.f, z);
-        redo = z != 0.f || z != z || tiny.x < kTinyBits || tiny.y < kTinyBits;
+        redo = z != 0.f || any_tiny(tiny);
     }
     if (__syncthreads_or(redo)) fp32_loop<A_KM, B_KM, BNT, DUAL>(g, m0, n0, t_begin, t_end, smem, acc);
     // accumulator (i, j, r): m = m0 + wm + 32 i + lane % 32,  n = n0 + wn + 32 j + 8 (r / 4) + 4 (lane / 32) + r % 4

@@ -1,5 +1,5 @@
-"""The fp32 matrix products' split-bf16 form (csrc/gemm_f32.hpp) at the places where it can go
-wrong, through the MLP entry points: K of a partial step only, of whole steps only and of both,
+"""The fp32 matrix products' split-bf16 form (csrc/gemm_f32.hpp, the tap kernel of
+csrc/conv3x3.hip) at the places where it can go wrong, through the MLP and conv entry points: K of a partial step only, of whole steps only and of both,
 output tiles with one row or column past a tile's edge; operands that the split cannot hold
 (under 2^-110), whose tiles are formed again in fp32; and operands that are not finite or
 round to infinity in bf16.  The bar is the fp32 one (1e-5 normwise against the Float32 oracle,
@@ -75,6 +75,72 @@ def test_split_product_non_finite(value):
     case.run_gpu()
     for (a, kind, _), want, dev in zip(args, host, case.dev):
         if kind != "Af":
+            continue
+        got = to_host(dev)
+        assert np.array_equal(np.isnan(got), np.isnan(want)), a
+        inf = np.isinf(want)
+        assert np.array_equal(np.isinf(got), inf) and np.array_equal(got[inf], want[inf]), a
+        ok = np.isfinite(want)
+        if np.any(want[ok]):
+            assert rel_err(got[ok], want[ok]) <= 1e-5, a
+
+
+def _conv(size):
+    N, C, K, H, W = size
+    sz = dict(loss=1, xp=(W + 2) * (H + 2) * C * N, w=9 * C * K, out=W * H * K * N)
+    return {k + suf: v for k, v in sz.items() for suf in ("", "b", "d", "bd")}, dict(zip(("i_nb", "i_c", "i_k", "i_h", "i_w"), size))
+
+
+@pytest.mark.parametrize("mode", ["b", "d", "hv"])
+@pytest.mark.parametrize("size", [(1, 15, 63, 3, 31), (1, 16, 64, 4, 32), (2, 17, 65, 9, 65), (1, 33, 5, 8, 33), (17, 3, 64, 61, 64)])
+def test_split_conv_edges(mode, size):
+    """One past and one short of a channel chunk, a row tile, a pixel tile; the last size has
+    enough tiles for the eight-row blocks, with a partial last one."""
+    shapes, ints = _conv(size)
+    s = 1.0 / np.sqrt(9.0 * size[1])
+    print(f"conv3x3_{mode} {size}", flush=True)
+    run_parity("conv3x3", mode, shapes, ints, precision="f32", scales={"w": s, "wd": s})
+
+
+@pytest.mark.parametrize("mode", ["b", "d", "hv"])
+@pytest.mark.parametrize("tiny", ["xp", "w"])
+def test_split_conv_tiny_operands(mode, tiny):
+    """Images (or weights) near 2^-122 against weights (images) near 2^110."""
+    size = (2, 18, 20, 6, 40)
+    shapes, ints = _conv(size)
+    s = 1.0 / np.sqrt(9.0 * size[1])
+    big = {"xp": "w", "w": "xp"}[tiny]
+    scales = {"w": s, "wd": s}
+    for a, e in ((tiny, -122), (big, 110)):
+        for suf in ("", "d"):
+            scales[a + suf] = scales.get(a + suf, 1.0) * 2.0 ** e
+    # keep every product of ordinary size: out ~ 2^-12, its seeds likewise
+    for a in ("out", "outb", "outd", "outbd"):
+        scales[a] = 2.0 ** -12
+    print(f"conv3x3_{mode} tiny {tiny}", flush=True)
+    run_parity("conv3x3", mode, shapes, ints, precision="f32", scales=scales)
+
+
+@pytest.mark.parametrize("value", [np.inf, 3.4e38])
+def test_split_conv_non_finite(value):
+    """One pixel that is not finite, or whose nearest bf16 is infinite."""
+    size = (1, 5, 9, 7, 40)
+    shapes, ints = _conv(size)
+    scales = {"w": 1e-20, "outb": 1e-20} if np.isfinite(value) else {}
+    lib = oracle_lib("conv3x3", "b", "f32")
+    args = make_args(lib, "conv3x3_b", shapes, ints, {}, "split-conv-non-finite", np.float32, None, scales)
+    for a, _, v in args:
+        if a == "xp":
+            v[2 * 9 * 42 + 4 * 42 + 20] = value
+        if a == "lossb" and np.isfinite(value):
+            v[:] = 1e-37
+    host = [v.copy() if isinstance(v, np.ndarray) else v for _, _, v in args]
+    lib.call("conv3x3_b", *host)
+    case = ParityCase("conv3x3", "b", args, (), "f32")
+    print(f"conv3x3_b one pixel {value}", flush=True)
+    case.run_gpu()
+    for (a, kind, _), want, dev in zip(args, host, case.dev):
+        if kind != "Af" or a == "loss":   # (the text's fp32 loss sum overflows where the fp64 one need not)
             continue
         got = to_host(dev)
         assert np.array_equal(np.isnan(got), np.isnan(want)), a
