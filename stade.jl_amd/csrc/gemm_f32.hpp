@@ -12,16 +12,18 @@
 // W1d * X + W1 * Xd is one launch.  A dual launch instead reads both segments in the same K
 // steps and writes two outputs, P = A0 B0 and Q = A0 B1 + A1 B0 (a product with its tangent).
 //
-// Arithmetic: six bf16 products of operands split into three bf16 parts (split_bf16.hpp).  What
-// is left is the rounding of the fp32 accumulation, once per instruction and 16 k, where
-// v_mfma_f32_32x32x2_f32 rounds every 2 k: against 64 bits (N(0, 1) times U(0, 1) operands) the
-// normwise error is 4.0e-7 at K = 784 and 9.9e-7 at K = 4096, of v_mfma_f32_32x32x2_f32 5.0e-7
-// and 1.1e-6.  The matrix cores run bf16 at 16 times the fp32 rate, so six products leave a
-// factor of 2.7.  Measured, us with fp32 MFMAs -> split: 1024 x 4096 x 784 64 -> 56, its dual
-// 179 -> 111; 1024 x 784 x 4096 (atomic K slices) 77 -> 58, dual 204 -> 137.  What bounds the
-// loop now is the splitting (12 vector instructions a pair of elements, 104 a wave and step
-// beside 24 MFMAs) and the LDS traffic that a block's two waves a SIMD do not hide wholly:
-// without the splitting the same loop runs at 270 TFLOP/s, with it at 180.
+// Arithmetic: six bf16 products of operands split into three bf16 parts (split_bf16.hpp).  A
+// step's products are summed from zero and then added to the tile's total: one rounding at the
+// total's size per 16 k, where v_mfma_f32_32x32x2_f32 rounds every 2 k (and where the six
+// products accumulated straight into the total would round six times).  Against 64 bits (N(0, 1)
+// times U(0, 1) operands) the normwise error is 1.4e-7 at K = 784 and 3.1e-7 at K = 4096; of
+// v_mfma_f32_32x32x2_f32 5.0e-7 and 1.1e-6, accumulated straight 4.0e-7 and 9.9e-7.
+// The matrix cores run bf16 at 16 times the fp32 rate, so six products leave a factor of 2.7.
+// Measured, us with fp32 MFMAs -> split: 1024 x 4096 x 784 64 -> 55, its dual 179 -> 121;
+// 1024 x 784 x 4096 (atomic K slices) 77 -> 60, dual 204 -> 149.  What bounds the loop now is
+// the splitting (12 vector instructions a pair of elements, 100 a wave and step beside 24 MFMAs)
+// and the loads and barriers that a block's two waves a SIMD do not hide wholly: without the
+// splitting and the loads the same loop runs at 270 TFLOP/s, with them at 165-180.
 // A block that meets an element the split cannot hold forms its tile again with fp32 matrix
 // instructions (fp32_loop): the results there are those of plain fp32.
 //
@@ -475,18 +477,31 @@ __device__ __forceinline__ void gemm_block(const Args& g, const Epi& epi, int bx
         constexpr bool WHOLE = decltype(whole_tag)::value;
         if (!WHOLE && !l0) return;
 #pragma unroll
-        for (int x = 0; x < 6; ++x)
+        for (int i = 0; i < 2; ++i) {
+            if (!WHOLE && i && !li) continue;
+            floatx16 v[NOP][NJ];
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int o = 0; o < NOP; ++o)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) v[o][j][r] = 0.f;
+#pragma unroll
+            for (int x = 0; x < 6; ++x)
 #pragma unroll
                 for (int j = 0; j < NJ; ++j) {
-                    if (!WHOLE && ((i && !li) || (j && !lj))) continue;
-                    acc[0][i][j] = mfma_bf16(fb[0][j][kSplitB[x]], fa[0][i][kSplitA[x]], acc[0][i][j]);
-                    if constexpr (DUAL) {
-                        acc[1][i][j] = mfma_bf16(fb[1][j][kSplitB[x]], fa[0][i][kSplitA[x]], acc[1][i][j]);
-                        acc[1][i][j] = mfma_bf16(fb[0][j][kSplitB[x]], fa[1][i][kSplitA[x]], acc[1][i][j]);
-                    }
+                    if (!WHOLE && j && !lj) continue;
+                    if constexpr (DUAL) v[1][j] = mfma_bf16(fb[1][j][kSplitB[x]], fa[0][i][kSplitA[x]], v[1][j]);
+                    v[0][j] = mfma_bf16(fb[0][j][kSplitB[x]], fa[0][i][kSplitA[x]], v[0][j]);
+                    if constexpr (DUAL) v[1][j] = mfma_bf16(fb[0][j][kSplitB[x]], fa[1][i][kSplitA[x]], v[1][j]);
                 }
+#pragma unroll
+            for (int o = 0; o < NOP; ++o)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[o][i][j][r] += v[o][j][r];
+        }
     };
     // step t (buffer p): its fragments from LDS, step t + 1 split and stored to the other
     // buffer, step t + 2's loads, t's MFMAs
