@@ -89,6 +89,24 @@ constexpr int FWD_S_NOTAPE = STADE_BURG_FS_NOTAPE, FWD_C_NOTAPE = STADE_BURG_FC_
 // waves) measured 2-3 % faster than one 1024-thread block.
 constexpr int BWD_T = STADE_BURG_BT, BWD_S = STADE_BURG_BS, BWD_T_HV = STADE_BURG_BT_HV, BWD_S_HV = STADE_BURG_BS_HV;
 
+// Small grids: one-wave blocks.  A launch's 32 steps are a serial chain, and below a few hundred
+// thousand cells the blocks above are too few to fill the chip, so a step's latency is what
+// counts: the block barrier, the edge values through LDS, and the cells that a thread updates one
+// after the other.  A block of one wave needs no barrier, and with a region of one slot no edge
+// values either (its ends are the region's, which no owned cell needs); its halo work is free on
+// idle SIMDs.  us a 32-step launch, one-wave form against the above:
+//   forward, tape        64 cells, 2 a lane   50000: 12 / 45 (tangent 14 / 75); 200000: 21 / 45 (53 / 76)
+//                        192 cells, 1 a lane  200000: 23 / 45 (32 / 76); 1000000: 60 / 56 (113 / 91)
+//   forward, no tape     64 cells, 2 a lane   7 launches: 50000: 64 / 105; 100000: 74 / 107; 200000: 114 / 114
+//   backward             128 cells            50000: 20 / 28; 200000: 24 / 29; 400000: 32 / 31
+//   backward, HVP        64 cells             50000: 23 / 33; 200000: 41 / 35
+// Two or more cells a lane with a tape store every other element, which costs more than the
+// edges save once the stores fill the memory system (192 / 4 at 400000: 123 / 46).
+constexpr int SMALL_FWD_N = 98304, SMALL_TAPE_N = 524288;  // up to: 64 / 2 a lane; with a tape 192 / 1
+constexpr int SMALL_FS = 64, SMALL_FC = 2, SMALL_TS = 192;
+constexpr int SMALL_BWD_N = 262144, SMALL_BWD_N_HV = 98304;
+constexpr int SMALL_BS = 128, SMALL_BS_HV = 64;
+
 struct Coef {
     double cadv, cdif, cadvd, cdifd;
 };
@@ -182,8 +200,12 @@ __global__ __launch_bounds__(T) void fwd_reg_kernel(const double* __restrict__ s
             }
         }
     };
-    publish(0);
-    __syncthreads();
+    // one wave with one slot: its ends are the region's, which no owned cell needs
+    constexpr bool ALONE = M == 1 && NWV == 1;
+    if constexpr (!ALONE) {
+        publish(0);
+        __syncthreads();
+    }
     for (int k = 0; k < nk; ++k) {
         const int buf = k & 1;
         // the state at the start of step t0 + k goes to tape row (t0 + k - row0) / every when
@@ -213,11 +235,11 @@ __global__ __launch_bounds__(T) void fwd_reg_kernel(const double* __restrict__ s
                 udn[i][j] = ud[i][j];
             }
             if (past(i)) continue;
-            const double eu = edge_at(buf, 0, i);
+            const double eu = ALONE ? 0.0 : edge_at(buf, 0, i);
             const double uw = from_west(u[i][C - 1], eu), ue = from_east(u[i][0], eu);
             double dw = 0.0, de = 0.0;
             if constexpr (TAN) {
-                const double ed = edge_at(buf, 1, i);
+                const double ed = ALONE ? 0.0 : edge_at(buf, 1, i);
                 dw = from_west(ud[i][C - 1], ed);
                 de = from_east(ud[i][0], ed);
             }
@@ -239,8 +261,10 @@ __global__ __launch_bounds__(T) void fwd_reg_kernel(const double* __restrict__ s
                 ud[i][j] = udn[i][j];
             }
         }
-        publish(buf ^ 1);
-        __syncthreads();
+        if constexpr (!ALONE) {
+            publish(buf ^ 1);
+            __syncthreads();
+        }
     }
 #pragma unroll
     for (int i = 0; i < M; ++i) {
@@ -701,7 +725,8 @@ int32_t forward(const double* src, const double* srcd, double* fin, double* find
     // the four-cell form also where the tape is sparse: at most one row a launch (the checkpoint
     // policy's first sweep, a row every `every` >= KMAX steps)
     const bool notape = tape == nullptr || every >= KMAX;
-    const unsigned nb = grid_for(n, notape ? FWD_S_NOTAPE : FWD_S);
+    const bool small = n <= SMALL_FWD_N, small_tape = !notape && n <= SMALL_TAPE_N;
+    const unsigned nb = grid_for(n, small ? SMALL_FS : notape ? FWD_S_NOTAPE : small_tape ? SMALL_TS : FWD_S);
     const double *cs = src, *csd = srcd;
     int64_t t0 = t_begin;
     int flip = 0;
@@ -710,7 +735,15 @@ int32_t forward(const double* src, const double* srcd, double* fin, double* find
         bool last = t0 + nk >= t_end;
         double* d = last ? fin : (flip ? Q : P);
         double* dd = last ? find : (flip ? Qd : Pd);
-        if (notape) {
+        if (small) {
+            STADE_TIMED(TAN ? "burgers1d_fwd_tan" : "burgers1d_fwd", stream,
+                        fwd_reg_kernel<TAN, SMALL_FS, 64, SMALL_FC><<<nb, 64, 0, stream>>>(cs, csd, d, dd, tape, taped, n, t0, nk, c, row0,
+                                                                                           every));
+        } else if (small_tape) {
+            STADE_TIMED(TAN ? "burgers1d_fwd_tan" : "burgers1d_fwd", stream,
+                        fwd_reg_kernel<TAN, SMALL_TS, 64, 1><<<nb, 64, 0, stream>>>(cs, csd, d, dd, tape, taped, n, t0, nk, c, row0,
+                                                                                    every));
+        } else if (notape) {
             STADE_TIMED(TAN ? "burgers1d_fwd_tan" : "burgers1d_fwd", stream,
                         fwd_reg_kernel<TAN, FWD_S_NOTAPE, BNT_NOTAPE, FWD_C_NOTAPE><<<nb, BNT_NOTAPE, 0, stream>>>(cs, csd, d, dd, tape, taped, n, t0, nk, c,
                                                                                         row0, every));
@@ -732,13 +765,24 @@ int32_t forward(const double* src, const double* srcd, double* fin, double* find
 int init_blocks(int64_t n) { return (int)grid_for((int)n, kInitBlockCells); }
 size_t bwd_offset(int64_t n) { return ((size_t)init_blocks(n) * 2 + 1023) / 1024 * 1024; }
 template <bool HV>
-int bwd_blocks(int64_t n) { return (int)grid_for((int)n, HV ? BWD_S_HV : BWD_S); }
+int bwd_blocks(int64_t n, bool small) {
+    return (int)grid_for((int)n, small ? (HV ? SMALL_BS_HV : SMALL_BS) : (HV ? BWD_S_HV : BWD_S));
+}
 // (every > 1: the checkpoint policy's reverse sweep, whose segments of `every` steps are
 // chunked separately)
 template <bool HV>
-int32_t check_partials(int64_t n, int64_t nrun, const char* fn, int64_t every = 1) {
+int64_t partials_needed(int64_t n, int64_t nrun, int64_t every, bool small) {
     const int64_t chunks = every > 1 ? (nrun + every - 1) / every * ((every + KMAX - 1) / KMAX) : (nrun + KMAX - 1) / KMAX;
-    const int64_t need = (int64_t)bwd_offset(n) + chunks * bwd_blocks<HV>(n) * (HV ? 4 : 2);
+    return (int64_t)bwd_offset(n) + chunks * bwd_blocks<HV>(n, small) * (HV ? 4 : 2);
+}
+// whether the reverse sweep takes the one-wave blocks (whose partials must fit, too)
+template <bool HV>
+bool small_backward(int64_t n, int64_t nrun, int64_t every) {
+    return n <= (HV ? SMALL_BWD_N_HV : SMALL_BWD_N) && partials_needed<HV>(n, nrun, every, true) <= kPartialSlots;
+}
+template <bool HV>
+int32_t check_partials(int64_t n, int64_t nrun, const char* fn, int64_t every = 1) {
+    const int64_t need = partials_needed<HV>(n, nrun, every, small_backward<HV>(n, nrun, every));
     if (need > kPartialSlots)
         return set_error(STADE_HIP_ERANGE, "%s: n * nsteps too large for the reduction workspace (%lld slots needed)", fn, (long long)need);
     return STADE_HIP_OK;
@@ -749,6 +793,7 @@ int32_t check_partials(int64_t n, int64_t nrun, const char* fn, int64_t every = 
 struct BwdState {
     double *cw, *cwd, *ow, *owd;
     int chunk;
+    bool small;  // one-wave blocks
 };
 
 // reverse sweep over steps t_hi, t_hi - 1, ..., t_lo, reading tape row t - row0 for step t;
@@ -758,14 +803,23 @@ int32_t backward_range(BwdState& st, double* ub, double* ubd, const double* tape
                        int64_t t_lo, int64_t row0, bool final, const Coef& c, double* pbwd, int* nparts, hipStream_t stream) {
     constexpr int S = HV ? BWD_S_HV : BWD_S, T = HV ? BWD_T_HV : BWD_T;
     constexpr int NV = HV ? 4 : 2;
-    const unsigned nb = grid_for(n, S);
+    constexpr int SS = HV ? SMALL_BS_HV : SMALL_BS;
+    const unsigned nb = grid_for(n, st.small ? SS : S);
     int64_t t = t_hi;
     while (t >= t_lo) {
         int nk = (int)((t - t_lo + 1) < KMAX ? (t - t_lo + 1) : KMAX);
         bool last = final && t - nk < t_lo;
         double* d = last ? ub : st.ow;
         double* dd = last ? ubd : st.owd;
-        if (nk == KMAX) {
+        if (nk == KMAX && st.small) {
+            STADE_TIMED(HV ? "burgers1d_bwd_hv" : "burgers1d_bwd", stream,
+                        bwd_reg_kernel<HV, SS, 2, 64><<<nb, 64, 0, stream>>>(st.cw, st.cwd, d, dd, tape, taped, n, t, c,
+                                                                         pbwd + (size_t)st.chunk * nb * NV, row0));
+        } else if (st.small) {
+            STADE_TIMED(HV ? "burgers1d_bwd_hv" : "burgers1d_bwd", stream,
+                        bwd_kernel<HV, SS, 64><<<nb, 64, 0, stream>>>(st.cw, st.cwd, d, dd, tape, taped, n, t, nk, c,
+                                                                   pbwd + (size_t)st.chunk * nb * NV, row0));
+        } else if (nk == KMAX) {
             STADE_TIMED(HV ? "burgers1d_bwd_hv" : "burgers1d_bwd", stream,
                         bwd_reg_kernel<HV, S, 2, T><<<nb, T, 0, stream>>>(st.cw, st.cwd, d, dd, tape, taped, n, t, c,
                                                                       pbwd + (size_t)st.chunk * nb * NV, row0));
@@ -789,7 +843,7 @@ int32_t backward_range(BwdState& st, double* ub, double* ubd, const double* tape
 template <bool HV>
 int32_t backward(double* w, double* wd, double* W2, double* W2d, double* ub, double* ubd, const double* tape, const double* taped,
                  int n, int64_t nrun, const Coef& c, double* pbwd, int* nparts, hipStream_t stream) {
-    BwdState st{w, wd, W2, W2d, 0};
+    BwdState st{w, wd, W2, W2d, 0, small_backward<HV>(n, nrun, 1)};
     return backward_range<HV>(st, ub, ubd, tape, taped, n, nrun - 1, 0, 0, true, c, pbwd, nparts, stream);
 }
 
@@ -802,7 +856,7 @@ template <bool HV>
 int32_t backward_ckpt(double* w, double* wd, double* W2, double* W2d, double* ub, double* ubd, const double* ck,
                       const double* ckd, double* seg, double* segd, double* R, int n, int64_t nrun, int every, const Coef& c,
                       double* pbwd, int* nparts, hipStream_t stream) {
-    BwdState st{w, wd, W2, W2d, 0};
+    BwdState st{w, wd, W2, W2d, 0, small_backward<HV>(n, nrun, every)};
     double *R1 = R, *R2 = R + n, *R1d = R + 2 * (size_t)n, *R2d = R + 3 * (size_t)n, *Rf = R + 4 * (size_t)n,
            *Rfd = R + 5 * (size_t)n;
     const int64_t nseg = (nrun + every - 1) / every;
