@@ -8,10 +8,10 @@
 // owner-computes gather (`cgen_gather_periodic_inverse` 7343-7529) for the adjoint scatter.
 //
 // Two kernel families:
-//   * wave-strip kernels: one wavefront per strip of 128 columns (n a multiple of 128, the
-//     benchmark grids; 16-byte accesses) or of 64 columns (n a multiple of 64 only) and a chunk
-//     of rows, no LDS and no barriers (described at their definition);
-//   * row-streaming kernels (every other n), described next.
+//   * wave-strip kernels: one wavefront per strip of 128 columns (n even, from 128 on, and 16-byte
+//     aligned arrays; 16-byte accesses) or of 64 columns (any n from 64 on) and a chunk of rows,
+//     no LDS and no barriers (described at their definition);
+//   * row-streaming kernels (n below 64, and sizes past the wave-strips' partials), described next.
 //
 // Row-streaming layout and work per launch:
 //   * A 256-thread block owns a strip of 256 columns (i) and a chunk of CH rows (j); thread t
@@ -345,7 +345,13 @@ __global__ __launch_bounds__(NT) void zero2_kernel(double* __restrict__ a, doubl
 }
 
 // ---------------------------------------------------------------------------------------
-// Wave-strip kernels: the fast path when n is a multiple of 64 and of the chunk height.
+// Wave-strip kernels: n >= 64.  RAG: n is not a multiple of the strip width or the chunk height;
+// the last strip and the last chunk are then moved back to end at n, and their columns and rows
+// that the strip or chunk before owns are computed again but neither stored nor summed.  Loads
+// stay unconditional.  Against the row-streaming kernels, which reload three to five rows per
+// row out of LDS behind a barrier (tangent / adjoint / HVP, us): n = 100 24 -> 13 / 35 -> 14 /
+// 52 -> 19, n = 1000 28 -> 15 / 41 -> 20 / 60 -> 34, n = 3000 72 -> 65 / 101 -> 78 / 207 -> 184,
+// n = 5000 179 -> 158 / 260 -> 219 / 520 -> 438.
 //
 // One wavefront owns a strip of 64 columns (lane l: column c0 + l) and a chunk of WCH rows,
 // and marches down it alone: no LDS, no barriers.  East / west neighbours come from the
@@ -401,27 +407,33 @@ __device__ __forceinline__ double step5dv(double up, double c, double dn, double
 
 struct WaveGeom {
     int c0, j0, oc, hc;
+    bool mine;  // RAG: this lane's column belongs to the strip
+    int r0;     // RAG: the chunk's first own row, from j0
 };
 // wave `wid` = strip wid % nstrips, chunk wid / nstrips of `rows` rows
+template <bool RAG>
 __device__ __forceinline__ WaveGeom wave_geom(int wid, int n, int nstrips, int rows) {
     const int lane = threadIdx.x & 63;
     WaveGeom g;
-    g.c0 = (wid % nstrips) * WS;
-    g.j0 = (wid / nstrips) * rows;
+    const int c = (wid % nstrips) * WS, j = (wid / nstrips) * rows;
+    g.c0 = RAG ? min(c, n - WS) : c;
+    g.j0 = RAG ? min(j, n - rows) : j;
     g.oc = g.c0 + lane;
+    g.mine = !RAG || g.oc >= c;
+    g.r0 = RAG ? j - g.j0 : 0;
     const int hoff = lane == 0 ? -2 : (lane == 1 ? -1 : (lane == 2 ? WS : WS + 1));
     g.hc = wrap1(g.c0 + hoff, n);
     return g;
 }
 
 // tangent: un, und of rows j0 .. j0+ROWS-1 from u, ud rows j0-1 .. j0+ROWS
-template <int ROWS, int D>
+template <int ROWS, int D, bool RAG>
 __global__ __launch_bounds__(256) void diffusion_d_wave(const double* __restrict__ u, const double* __restrict__ ud,
                                                         double* __restrict__ un, double* __restrict__ und, int n,
                                                         int nstrips, int nwaves, double* partials) {
     const int wid = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (wid >= nwaves) return;  // whole waves only; the kernel has no barrier
-    const WaveGeom g = wave_geom(wid, n, nstrips, ROWS);
+    const WaveGeom g = wave_geom<RAG>(wid, n, nstrips, ROWS);
     double U[ROWS + 2], H[ROWS + 2], UD[ROWS + 2], HD[ROWS + 2];  // row q at index q + 1
     auto load = [&](int q) {
         const size_t rb = (size_t)wrap1(g.j0 + q, n) * n;
@@ -443,10 +455,12 @@ __global__ __launch_bounds__(256) void diffusion_d_wave(const double* __restrict
         const double vd =
             step5dv(UD[i - 1], UD[i], UD[i + 1], from_west(UD[i], lane_val(HD[i], 1)), from_east(UD[i], lane_val(HD[i], 2)));
         const size_t gi = (size_t)(g.j0 + r) * n + g.oc;
-        und[gi] = vd;
-        un[gi] = v;
-        acc[1] += (2.0 * v) * vd;
-        acc[0] += v * v;
+        if (!RAG || (g.mine && r >= g.r0)) {
+            und[gi] = vd;
+            un[gi] = v;
+            acc[1] += (2.0 * v) * vd;
+            acc[0] += v * v;
+        }
     }
     acc[0] = wave_sum(acc[0]);
     acc[1] = wave_sum(acc[1]);
@@ -458,7 +472,7 @@ __global__ __launch_bounds__(256) void diffusion_d_wave(const double* __restrict
 
 // adjoint pass 1 (HV = false) and its tangent (HV = true): un (+ und) of the wave's rows,
 // loss partials, and the gather of w = unb + (2 un) lossb (+ wd) into ub (+ ubd)
-template <bool HV, int ROWS, int D>
+template <bool HV, int ROWS, int D, bool RAG>
 __global__ __launch_bounds__(256) void diffusion_b_wave(const double* __restrict__ u, const double* __restrict__ ud,
                                                         double* __restrict__ un, double* __restrict__ und,
                                                         const double* __restrict__ unb, const double* __restrict__ unbd,
@@ -467,7 +481,7 @@ __global__ __launch_bounds__(256) void diffusion_b_wave(const double* __restrict
                                                         int n, int nstrips, int nwaves, double* partials) {
     const int wid = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (wid >= nwaves) return;  // whole waves only; the kernel has no barrier
-    const WaveGeom g = wave_geom(wid, n, nstrips, ROWS);
+    const WaveGeom g = wave_geom<RAG>(wid, n, nstrips, ROWS);
     const double lb = lossb[0];
     const double lbd = HV ? lossbd[0] : 0.0;
     // u rows -2 .. ROWS+1 at index q + 2; unb rows -1 .. ROWS at q + 1; ub rows 0 .. ROWS-1
@@ -526,7 +540,7 @@ __global__ __launch_bounds__(256) void diffusion_b_wave(const double* __restrict
             WDw[b] = lane_val(BHD[b], 1) + (lb * (2.0 * vdw) + (2.0 * vw) * lbd);
             WDe[b] = lane_val(BHD[b], 2) + (lb * (2.0 * vde) + (2.0 * ve) * lbd);
         }
-        if (q >= 0 && q < ROWS) {
+        if (q >= 0 && q < ROWS && (!RAG || (g.mine && q >= g.r0))) {
             const size_t gi = (size_t)(g.j0 + q) * n + g.oc;
             if constexpr (HV) {
                 und[gi] = vd;
@@ -547,6 +561,7 @@ __global__ __launch_bounds__(256) void diffusion_b_wave(const double* __restrict
         a = a + 0.1 * Wo[b - 1];
         a = a + 4.0 * -(0.1 * c);
         const size_t gi = (size_t)(g.j0 + r) * n + g.oc;
+        const bool store = !RAG || (g.mine && r >= g.r0);
         if constexpr (HV) {
             const double cd = WDo[b];
             double ad = cd;
@@ -555,9 +570,9 @@ __global__ __launch_bounds__(256) void diffusion_b_wave(const double* __restrict
             ad = ad + 0.1 * WDo[b + 1];
             ad = ad + 0.1 * WDo[b - 1];
             ad = ad + 4.0 * -(0.1 * cd);
-            ubd[gi] = UBD[r] + ad;
+            if (store) ubd[gi] = UBD[r] + ad;
         }
-        ub[gi] = UB[r] + a;
+        if (store) ub[gi] = UB[r] + a;
     };
 #pragma unroll
     for (int q = -2; q <= 1; ++q) load_u(q);
@@ -618,13 +633,19 @@ void with_rows(int rows, F&& f) {
 
 struct WaveGeom2 {
     int lane, c0, j0, oc, hc;
+    bool mine;  // RAG: this lane's pair belongs to the strip
+    int r0;     // RAG: the chunk's first own row, from j0
 };
+template <bool RAG>
 __device__ __forceinline__ WaveGeom2 wave_geom2(int wid, int n, int nstrips, int rows) {
     WaveGeom2 g;
     g.lane = threadIdx.x & 63;
-    g.c0 = (wid % nstrips) * WS2;
-    g.j0 = (wid / nstrips) * rows;
+    const int c = (wid % nstrips) * WS2, j = (wid / nstrips) * rows;
+    g.c0 = RAG ? min(c, n - WS2) : c;  // (n is even: pairs stay pairs)
+    g.j0 = RAG ? min(j, n - rows) : j;
     g.oc = g.c0 + 2 * g.lane;
+    g.mine = !RAG || g.oc >= c;
+    g.r0 = RAG ? j - g.j0 : 0;
     g.hc = wrap1(g.c0 + (g.lane == 0 ? -2 : (g.lane == 1 ? -1 : (g.lane == 2 ? WS2 : WS2 + 1))), n);
     return g;
 }
@@ -647,7 +668,7 @@ __device__ __forceinline__ double2 step_pair(double2 up, double2 c, double2 dn, 
 }
 
 // tangent: un, und of rows j0 .. j0+ROWS-1 from u, ud rows j0-1 .. j0+ROWS
-template <int ROWS, int D>
+template <int ROWS, int D, bool RAG>
 __global__ __launch_bounds__(256) void diffusion_d_wave2(const double* __restrict__ u, const double* __restrict__ ud,
                                                          double* __restrict__ un, double* __restrict__ und, int n,
                                                          int nstrips, int nwaves, double* partials) {
@@ -655,7 +676,7 @@ __global__ __launch_bounds__(256) void diffusion_d_wave2(const double* __restric
     const int wid = blockIdx.x * 4 + (threadIdx.x >> 6);
     double acc[2] = {0.0, 0.0};
     if (wid < nwaves) {  // whole waves; the four of a block meet at the barrier below
-        const WaveGeom2 g = wave_geom2(wid, n, nstrips, ROWS);
+        const WaveGeom2 g = wave_geom2<RAG>(wid, n, nstrips, ROWS);
         const double2* __restrict__ u2 = reinterpret_cast<const double2*>(u);
         const double2* __restrict__ ud2 = reinterpret_cast<const double2*>(ud);
         double2* __restrict__ un2 = reinterpret_cast<double2*>(un);
@@ -679,12 +700,14 @@ __global__ __launch_bounds__(256) void diffusion_d_wave2(const double* __restric
             const double2 v = step_pair<false>(U[i - 1], U[i], U[i + 1], lane_val(H[i], 1), lane_val(H[i], 2));
             const double2 vd = step_pair<true>(UD[i - 1], UD[i], UD[i + 1], lane_val(HD[i], 1), lane_val(HD[i], 2));
             const size_t gp = pair_of((size_t)(g.j0 + r) * n, g.oc);
-            nt_store2(vd, &und2[gp]);
-            nt_store2(v, &un2[gp]);
-            acc[1] += (2.0 * v.x) * vd.x;
-            acc[0] += v.x * v.x;
-            acc[1] += (2.0 * v.y) * vd.y;
-            acc[0] += v.y * v.y;
+            if (!RAG || (g.mine && r >= g.r0)) {
+                nt_store2(vd, &und2[gp]);
+                nt_store2(v, &un2[gp]);
+                acc[1] += (2.0 * v.x) * vd.x;
+                acc[0] += v.x * v.x;
+                acc[1] += (2.0 * v.y) * vd.y;
+                acc[0] += v.y * v.y;
+            }
         });
     }
     // one partial pair per block: its four waves' sums added in wave order
@@ -693,7 +716,7 @@ __global__ __launch_bounds__(256) void diffusion_d_wave2(const double* __restric
 
 // adjoint pass 1 (HV = false) and its tangent (HV = true): un (+ und) of the wave's rows,
 // loss partials, and the gather of w = unb + (2 un) lossb (+ wd) into ub (+ ubd)
-template <bool HV, int ROWS, int D>
+template <bool HV, int ROWS, int D, bool RAG>
 __global__ __launch_bounds__(256) void diffusion_b_wave2(const double* __restrict__ u, const double* __restrict__ ud,
                                                          double* __restrict__ un, double* __restrict__ und,
                                                          const double* __restrict__ unb, const double* __restrict__ unbd,
@@ -704,7 +727,7 @@ __global__ __launch_bounds__(256) void diffusion_b_wave2(const double* __restric
     const int wid = blockIdx.x * 4 + (threadIdx.x >> 6);
     double acc[2] = {0.0, 0.0};
     if (wid < nwaves) {  // whole waves; the four of a block meet at the barrier below
-        const WaveGeom2 g = wave_geom2(wid, n, nstrips, ROWS);
+        const WaveGeom2 g = wave_geom2<RAG>(wid, n, nstrips, ROWS);
         const double lb = lossb[0];
         const double lbd = HV ? lossbd[0] : 0.0;
         const double2* __restrict__ u2 = reinterpret_cast<const double2*>(u);
@@ -775,7 +798,7 @@ __global__ __launch_bounds__(256) void diffusion_b_wave2(const double* __restric
                 WDw[b] = lane_val(BHD[b], 1) + (lb * (2.0 * vdw) + (2.0 * vw) * lbd);
                 WDe[b] = lane_val(BHD[b], 2) + (lb * (2.0 * vde) + (2.0 * ve) * lbd);
             }
-            if (q >= 0 && q < ROWS) {
+            if (q >= 0 && q < ROWS && (!RAG || (g.mine && q >= g.r0))) {
                 const size_t gp = pair_of((size_t)(g.j0 + q) * n, g.oc);
                 if constexpr (HV) {
                     nt_store2(vd, &und2[gp]);
@@ -800,18 +823,19 @@ __global__ __launch_bounds__(256) void diffusion_b_wave2(const double* __restric
         auto gather = [&](int r) {
             const int b = r + 1;
             const size_t gp = pair_of((size_t)(g.j0 + r) * n, g.oc);
+            const bool store = !RAG || (g.mine && r >= g.r0);
             if constexpr (HV) {
                 const double2 c = WDo[b];
                 double2 o;
                 o.x = UBD[r].x + gather1(c.x, c.y, from_west(c.y, WDw[b]), WDo[b + 1].x, WDo[b - 1].x);
                 o.y = UBD[r].y + gather1(c.y, from_east(c.x, WDe[b]), c.x, WDo[b + 1].y, WDo[b - 1].y);
-                nt_store2(o, &ubd2[gp]);
+                if (store) nt_store2(o, &ubd2[gp]);
             }
             const double2 c = Wo[b];
             double2 o;
             o.x = UB[r].x + gather1(c.x, c.y, from_west(c.y, Ww[b]), Wo[b + 1].x, Wo[b - 1].x);
             o.y = UB[r].y + gather1(c.y, from_east(c.x, We[b]), c.x, Wo[b + 1].y, Wo[b - 1].y);
-            nt_store2(o, &ub2[gp]);
+            if (store) nt_store2(o, &ub2[gp]);
         };
 #pragma unroll
         for (int q = -2; q <= 1; ++q) load_u(q);
@@ -837,23 +861,46 @@ __global__ __launch_bounds__(256) void diffusion_b_wave2(const double* __restric
     }
 }
 
+constexpr int64_t kNoAllocPartials = 131072;  // doubles of the allocation-free adjoint's scratch
+
 struct WaveGrid {
     int nstrips, nwaves, blocks;
+    bool rag;
 };
+WaveGrid wave_grid(int64_t n, int width, int rows) {
+    const int nstrips = (int)((n + width - 1) / width), nwaves = nstrips * (int)((n + rows - 1) / rows);
+    return WaveGrid{nstrips, nwaves, (nwaves + 3) / 4, n % width != 0 || n % rows != 0};
+}
 // the 128-column kernels move 16-byte pairs: every array they touch must be 16-byte aligned
-// (an array that is a view into a larger allocation may be 8-byte aligned only)
+// (an array that is a view into a larger allocation may be 8-byte aligned only), and so must
+// every row (n even).  Ragged sizes take either kind of strip only where their partials fit
+// the allocation-free scratch (n <= 16384, so that one rule holds for every entry point).
+constexpr int64_t kRaggedMax = 16384;
 bool pairs_ok(int64_t n, std::initializer_list<const void*> arrays) {
-    if (n % WS2 != 0) return false;
+    if (n % WS2 != 0 && (n % 2 != 0 || n < WS2 || n > kRaggedMax)) return false;
     for (const void* p : arrays)
         if (reinterpret_cast<uintptr_t>(p) & 15) return false;
     return true;
 }
-// the wave-strip path applies when n is a multiple of the strip width (and so of the rows
-// per wave)
-bool wave_path(int64_t n) { return n >= WS && n % WS == 0; }
-WaveGrid wave_grid_of(int64_t n, int rows) {
-    const int nstrips = (int)(n / WS), nwaves = nstrips * (int)(n / rows);
-    return WaveGrid{nstrips, nwaves, (nwaves + 3) / 4};
+bool wave_path(int64_t n) { return n >= WS && (n % WS == 0 || n <= kRaggedMax); }
+// rows of a 64-column strip's chunk at ragged sizes: 16 rows for the waves that a smaller grid
+// needs, 32 from where the grid fills the chip with those (fewer halo rows, half the partials).
+// Adjoint, 16 against 32 rows: n = 1001 18.3 / 21.4 us, 3001 99 / 101, 4095 181 / 177,
+// 7001 533 / 517 (the row-streaming kernels: 40.8, 104, 179, 528)
+int rows_ragged(int64_t n) { return n < 3584 ? 16 : 32; }
+WaveGrid wave_grid64(int64_t n, int rows) { return wave_grid(n, WS, n % WS == 0 ? rows : rows_ragged(n)); }
+// calls f with whether the strips are ragged as a compile-time constant
+template <typename F>
+void with_rag(bool rag, F&& f) {
+    if (rag) f(std::true_type{});
+    else f(std::false_type{});
+}
+// the 64-column strips: f with the chunk height (`rows` at multiples of 64) and raggedness
+template <int ROWS, typename F>
+void with_strips64(int64_t n, F&& f) {
+    if (n % WS == 0) return f(std::integral_constant<int, ROWS>{}, std::false_type{});
+    if (rows_ragged(n) == 16) f(std::integral_constant<int, 16>{}, std::true_type{});
+    else f(std::integral_constant<int, 32>{}, std::true_type{});
 }
 
 int32_t check_n(int64_t n, const char* fn) {
@@ -880,8 +927,8 @@ Grid grid_of(int64_t n) {
 // the adjoint's reduction partials: one per block of pass 1 (one per wave on the 64-column
 // strips)
 int64_t adjoint_partials(int64_t n, bool pairs) {
-    if (pairs) return ((n / WS2) * (n / rows_b2(n)) + 3) / 4;
-    if (wave_path(n)) return (n / WS) * (n / WCH);
+    if (pairs) return wave_grid(n, WS2, rows_b2(n)).blocks;
+    if (wave_path(n)) return wave_grid64(n, WCH).nwaves;
     const Grid g = grid_of(n);
     return g.blocks;
 }
@@ -893,18 +940,20 @@ int32_t adjoint(double* loss, const double* lossb, const double* u, double* ub, 
                 double* partials, hipStream_t stream) {
     int nparts;
     if (pairs_ok(n, {u, un, unb, ub})) {
-        const int rows = rows_b2(n), nstrips = (int)(n / WS2), nwaves = nstrips * (int)(n / rows);
-        STADE_TIMED("diffusion2d_b", stream, with_rows<64>(rows, [&](auto rc) {
-                        diffusion_b_wave2<false, decltype(rc)::value, WD><<<(nwaves + 3) / 4, 256, 0, stream>>>(
-                            u, nullptr, un, nullptr, unb, nullptr, ub, nullptr, lossb, nullptr, (int)n, nstrips, nwaves, partials);
-                    }));
+        const int rows = rows_b2(n);
+        const WaveGrid w = wave_grid(n, WS2, rows);
+        STADE_TIMED("diffusion2d_b", stream, with_rag(w.rag, [&](auto rag) { with_rows<64>(rows, [&](auto rc) {
+                        diffusion_b_wave2<false, decltype(rc)::value, WD, decltype(rag)::value><<<w.blocks, 256, 0, stream>>>(
+                            u, nullptr, un, nullptr, unb, nullptr, ub, nullptr, lossb, nullptr, (int)n, w.nstrips, w.nwaves, partials);
+                    }); }));
         STADE_LAUNCHED("diffusion_b_wave2");
-        nparts = (nwaves + 3) / 4;
+        nparts = w.blocks;
     } else if (wave_path(n)) {
-        const WaveGrid w = wave_grid_of(n, WCH);
-        STADE_TIMED("diffusion2d_b", stream,
-                    diffusion_b_wave<false, WCH, WD><<<w.blocks, 256, 0, stream>>>(u, nullptr, un, nullptr, unb, nullptr, ub, nullptr,
-                                                                              lossb, nullptr, (int)n, w.nstrips, w.nwaves, partials));
+        const WaveGrid w = wave_grid64(n, WCH);
+        STADE_TIMED("diffusion2d_b", stream, with_strips64<WCH>(n, [&](auto rc, auto rag) {
+                        diffusion_b_wave<false, decltype(rc)::value, WD, decltype(rag)::value><<<w.blocks, 256, 0, stream>>>(
+                            u, nullptr, un, nullptr, unb, nullptr, ub, nullptr, lossb, nullptr, (int)n, w.nstrips, w.nwaves, partials);
+                    }));
         STADE_LAUNCHED("diffusion_b_wave");
         nparts = w.nwaves;
     } else {
@@ -928,7 +977,6 @@ int32_t adjoint(double* loss, const double* lossb, const double* u, double* ub, 
 // code never passes `scratch` itself (in host code the name is a stand-in, not a device
 // address): each device's address is looked up once with hipGetSymbolAddress and kept.
 // ------------------------------------------------------------------------------------------
-constexpr int64_t kNoAllocPartials = 131072;  // 1 MiB of doubles
 static __device__ __align__(256) double scratch[kNoAllocPartials];
 static std::mutex g_scratch_mu;
 static double* g_scratch_ptr[64];
@@ -990,17 +1038,20 @@ int32_t stade_hip_diffusion2d_d(double* loss, double* lossd, const double* u, co
     if (!ws) return STADE_HIP_ENOMEM;
     int nparts;
     if (pairs_ok(n, {u, ud, un, und})) {
-        const int rows = rows_d2(n), nstrips = (int)(n / WS2), nwaves = nstrips * (int)(n / rows);
-        STADE_TIMED("diffusion2d_d", stream, with_rows<32>(rows, [&](auto rc) {
-                        diffusion_d_wave2<decltype(rc)::value, WD><<<(nwaves + 3) / 4, 256, 0, stream>>>(
-                            u, ud, un, und, (int)n, nstrips, nwaves, ws->partials);
-                    }));
+        const int rows = rows_d2(n);
+        const WaveGrid w = wave_grid(n, WS2, rows);
+        STADE_TIMED("diffusion2d_d", stream, with_rag(w.rag, [&](auto rag) { with_rows<32>(rows, [&](auto rc) {
+                        diffusion_d_wave2<decltype(rc)::value, WD, decltype(rag)::value><<<w.blocks, 256, 0, stream>>>(
+                            u, ud, un, und, (int)n, w.nstrips, w.nwaves, ws->partials);
+                    }); }));
         STADE_LAUNCHED("diffusion_d_wave2");
-        nparts = (nwaves + 3) / 4;
+        nparts = w.blocks;
     } else if (wave_path(n)) {
-        const WaveGrid w = wave_grid_of(n, WCH);
-        STADE_TIMED("diffusion2d_d", stream,
-                    diffusion_d_wave<WCH, WD><<<w.blocks, 256, 0, stream>>>(u, ud, un, und, (int)n, w.nstrips, w.nwaves, ws->partials));
+        const WaveGrid w = wave_grid64(n, WCH);
+        STADE_TIMED("diffusion2d_d", stream, with_strips64<WCH>(n, [&](auto rc, auto rag) {
+                        diffusion_d_wave<decltype(rc)::value, WD, decltype(rag)::value><<<w.blocks, 256, 0, stream>>>(u, ud, un, und, (int)n, w.nstrips,
+                                                                                                     w.nwaves, ws->partials);
+                    }));
         STADE_LAUNCHED("diffusion_d_wave");
         nparts = w.nwaves;
     } else {
@@ -1038,18 +1089,20 @@ int32_t stade_hip_diffusion2d_hv(double* loss, const double* lossb, const double
     if (!ws) return STADE_HIP_ENOMEM;
     int nparts;
     if (pairs_ok(n, {u, ud, un, und, unb, unbd, ub, ubd})) {
-        const int rows = rows_hv2(n), nstrips = (int)(n / WS2), nwaves = nstrips * (int)(n / rows);
-        STADE_TIMED("diffusion2d_hv", stream, with_rows<32>(rows, [&](auto rc) {
-                        diffusion_b_wave2<true, decltype(rc)::value, WD2_HV><<<(nwaves + 3) / 4, 256, 0, stream>>>(
-                            u, ud, un, und, unb, unbd, ub, ubd, lossb, lossbd, (int)n, nstrips, nwaves, ws->partials);
-                    }));
+        const int rows = rows_hv2(n);
+        const WaveGrid w = wave_grid(n, WS2, rows);
+        STADE_TIMED("diffusion2d_hv", stream, with_rag(w.rag, [&](auto rag) { with_rows<32>(rows, [&](auto rc) {
+                        diffusion_b_wave2<true, decltype(rc)::value, WD2_HV, decltype(rag)::value><<<w.blocks, 256, 0, stream>>>(
+                            u, ud, un, und, unb, unbd, ub, ubd, lossb, lossbd, (int)n, w.nstrips, w.nwaves, ws->partials);
+                    }); }));
         STADE_LAUNCHED("diffusion_b_wave2<hv>");
-        nparts = (nwaves + 3) / 4;
+        nparts = w.blocks;
     } else if (wave_path(n)) {
-        const WaveGrid w = wave_grid_of(n, WCH_HV);
-        STADE_TIMED("diffusion2d_hv", stream,
-                    diffusion_b_wave<true, WCH_HV, WD_HV><<<w.blocks, 256, 0, stream>>>(u, ud, un, und, unb, unbd, ub, ubd, lossb, lossbd,
-                                                                                (int)n, w.nstrips, w.nwaves, ws->partials));
+        const WaveGrid w = wave_grid64(n, WCH_HV);
+        STADE_TIMED("diffusion2d_hv", stream, with_strips64<WCH_HV>(n, [&](auto rc, auto rag) {
+                        diffusion_b_wave<true, decltype(rc)::value, WD_HV, decltype(rag)::value><<<w.blocks, 256, 0, stream>>>(
+                            u, ud, un, und, unb, unbd, ub, ubd, lossb, lossbd, (int)n, w.nstrips, w.nwaves, ws->partials);
+                    }));
         STADE_LAUNCHED("diffusion_b_wave<hv>");
         nparts = w.nwaves;
     } else {
