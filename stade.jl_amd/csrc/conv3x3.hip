@@ -13,9 +13,8 @@
 //   adjoint  g = outb + (0.5 (2 out)) lossb  (the accumulated outb, then reset to 0)
 //            wb[co][c][ky][kx] += sum_{n,y,x} g[n][co][y][x] xp[n][c][y+ky][x+kx]
 //            xpb[n][c][yp][xq] += sum_{co,ky,kx} w[co][c][ky][kx] g[n][co][yp-ky][xq-kx]
-// All three run on the matrix cores as implicit GEMMs (the tap kernel's by split bf16, the
-// weight gradient's by v_mfma_f32_32x32x2_f32): no im2col buffer; each block stages an input patch and a weight slice in LDS and the MFMA
-// operands are read from the patch at tap-shifted offsets.
+// All three run on the matrix cores as implicit GEMMs by split bf16, with no im2col buffer: each
+// block stages its operands in LDS, and the taps read them there at shifted offsets.
 //   tap_kernel    forward (and the tangent's two products) and the interior of xpb, which
 //                 is the same shifted product on g with flipped, transposed weights
 //   border_kernel the one-cell frame of xpb (taps that land on the zero padding): four 1-D
@@ -632,134 +631,236 @@ __global__ __launch_bounds__(NT) void border_kernel(BorderArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------
-// weight gradient: part[split][ct][kt][t][ci][co] = sum over the split's pixel tiles of
+// weight gradient: part[split][ct][kt][t][ci][co] = sum over the split's pixel rows of
 //   sum_p sum_{pixel} x_p[n][c][y+ky][x+kx] * g_p[n][co][y][x]
-// Block: 256 threads, a 64 (c) x 64 (co) slab of all 9 taps; wave (wa, wb) owns the
-// 32 x 32 quarter (c half wa, co half wb) of every tap: 9 accumulator tiles.  Pixel tiles of
-// 32 x 2 pixels: the (2+2) x (32+2) patch of 64 channels and the 64 x 64 g tile are staged in
-// LDS (next tile prefetched into registers); the MFMA k pair is a pair of adjacent pixels.
+// Block: 256 threads, a 64 (c) x 64 (co) slab of all 9 taps; wave (wa, wb) owns the 32 x 32
+// quarter (c half wa, co half wb) of every tap: 9 accumulator tiles.  The pixels are the
+// product's k: strips of 8 S columns, walked down row by row.  Each row's x (64 channels) and g
+// (64 channels) are split into bf16 parts (split_bf16.hpp) once and kept in LDS, x in a ring of
+// four rows, so that a row is read from memory once for its three ky.
+// Cell s of a row holds the eight pixels s, s + S, .., s + 7 S of one channel: a tap's shift by
+// kx is then another cell and not a misaligned read (S + 2 cells hold all three shifts, a quarter
+// of the row twice), and cells 2 ks, 2 ks + 1 are one k step of 16 pixels.  A cell plane is 65
+// channels wide so that the staging threads, consecutive in s, write to different banks.
+// A row's products (24 a tap) are summed from zero and then added to the total, which rounds
+// once a row there where v_mfma_f32_32x32x2_f32 rounds every two pixels.  The next row is
+// loaded, split and stored between the MFMAs.  A block that meets an element which the split
+// cannot hold forms its sums again in fp32 with operands straight from memory.
+// Measured, us with fp32 MFMAs (tiles of 32 x 2 pixels, each row staged twice) -> split:
+// 8 x 64 -> 64 x 256^2 390 -> 235 (165 TFLOP/s; the MFMAs alone 93 at the bf16 peak).  One wave
+// a SIMD (453 registers): what the MFMAs do not hide is the LDS reads (120 of 16 bytes a wave and
+// row beside 216 MFMAs) and the two barriers a row.
 // ------------------------------------------------------------------------------------------
-constexpr int WTX = 32, WTY = 2;
-constexpr int XPX = WTX + 2;                   // 34
-constexpr int XPL = XPX * (WTY + 2);           // 136 floats of one channel's patch
-constexpr int XPP = XPL + 1;                   // LDS plane stride (odd)
-constexpr int GPX = WTX * WTY, GPP = GPX + 1;  // 64 pixels, LDS row stride 65
-constexpr int XSZ = 64 * XPP, GSZ = 64 * GPP;
+constexpr int WGP = 65;  // channels of a cell plane, padded
 
 struct WgArgs {
     const float* x[2];  // xp-shaped
     const float* g[2];  // out-shaped
     int N, C, K, H, W;
-    int ntx, nty, ntiles;  // pixel tiles of one (x, g) pair
-    int npairs;            // NPR = 1: tiles [p * ntiles, (p + 1) * ntiles) use pair p
+    int ntx;            // strips
+    long nrows;         // pixel rows of all strips, images and (x, g) pairs
     float* part;
 };
 
-template <int NPR>
-__global__ __launch_bounds__(NT) void wgrad_kernel(WgArgs a) {
-    constexpr int XLD = 64 * XPL / NT;  // 34
-    constexpr int GLD = 64 * GPX / NT;  // 16
-    static_assert(64 * XPL % NT == 0 && 64 * GPX % NT == 0, "wgrad stage");
-    __shared__ float lds[NPR * (XSZ + GSZ)];
-    float* Xs = lds;
-    float* Gs = lds + NPR * XSZ;
+// a block's pixel rows: [lo, hi) of the nrows, in the order pair, image, strip, y
+struct WgRow {
+    int pr, n, x0, y;
+    __device__ __forceinline__ WgRow(const WgArgs& a, long r, int width) {
+        const long q = r / a.H;
+        y = (int)(r - q * a.H);
+        const long i = q / a.ntx;
+        x0 = (int)(q - i * a.ntx) * width;
+        pr = i >= a.N;
+        n = (int)(i - (long)pr * a.N);
+    }
+};
 
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+template <int S>
+__global__ __launch_bounds__(NT) void wgrad_kernel(WgArgs a) {
+    constexpr int XC = 64 * (S + 2), GC = 64 * S;                    // cells of a row
+    constexpr int NX = (XC + NT - 1) / NT, NG = (GC + NT - 1) / NT;  // ... of a thread
+    constexpr int XPART = (S + 2) * WGP, GPART = S * WGP;            // ... of a part, padded
+    __shared__ u32x4 xs[4][3 * XPART];
+    __shared__ u32x4 gs[3 * GPART];
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, l32 = lane & 31;
     const int ktn = (a.K + 63) / 64;
     const int ct = blockIdx.x / ktn, kt = blockIdx.x - ct * ktn;
     const int c0 = ct * 64, k0 = kt * 64;
     const int wa = wave & 1, wb = wave >> 1;
     const int Hp = a.H + 2, Wp = a.W + 2;
+    const int xplane = Hp * Wp, gplane = a.H * a.W;
+    const long lo = a.nrows * blockIdx.y / gridDim.y, hi = a.nrows * (blockIdx.y + 1) / gridDim.y;
 
-    float xr[NPR][XLD], gr[NPR][GLD];
-    auto load = [&](int tile) {
-        // NPR = 1 with two pairs: the pair is uniform over the block's tile
-        const int pr = NPR == 1 && tile >= a.ntiles ? 1 : 0;
-        tile -= pr * a.ntiles;
-        const float* xs[2] = {a.x[pr], a.x[1]};
-        const float* gs[2] = {a.g[pr], a.g[1]};
-        const int xt = tile % a.ntx;
-        const int rest = tile / a.ntx;
-        const int yt = rest % a.nty, n = rest / a.nty;
-        const int x0 = xt * WTX, y0 = yt * WTY;
-#pragma unroll
-        for (int p = 0; p < NPR; ++p) {
-#pragma unroll
-            for (int q = 0; q < XLD; ++q) {
-                const int f = threadIdx.x + q * NT;
-                const int ci = f / XPL, e = f - ci * XPL;
-                const int ty = e / XPX, tx = e - ty * XPX;
-                const int c = c0 + ci, yy = y0 + ty, xx = x0 + tx;
-                xr[p][q] = (c < a.C && yy < Hp && xx < Wp) ? xs[p][((long)(n * a.C + c) * Hp + yy) * Wp + xx] : 0.f;
-            }
-#pragma unroll
-            for (int q = 0; q < GLD; ++q) {
-                const int f = threadIdx.x + q * NT;
-                const int co = f / GPX, px = f - co * GPX;
-                const int k = k0 + co, yy = y0 + px / WTX, xx = x0 + px % WTX;
-                gr[p][q] = (k < a.K && yy < a.H && xx < a.W) ? gs[p][((long)(n * a.K + k) * a.H + yy) * a.W + xx] : 0.f;
-            }
-        }
+    // Buffer loads: a scalar resource per image, the row as a scalar offset, channel and pixel
+    // as the lane's; an element outside reads an offset past the resource, which returns 0.
+    // (The host keeps one image under 2^31 bytes.)
+    constexpr uint32_t kPast = 0x80000000u;
+    __amdgpu_buffer_rsrc_t rx, rg;
+    auto image = [&](const WgRow& w) {
+        rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.x[w.pr] + (long)w.n * a.C * xplane), (short)0,
+                                               (uint32_t)((long)a.C * xplane * 4), kBufWord3);
+        rg = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.g[w.pr] + (long)w.n * a.K * gplane), (short)0,
+                                               (uint32_t)((long)a.K * gplane * 4), kBufWord3);
     };
-    auto store = [&]() {
-#pragma unroll
-        for (int p = 0; p < NPR; ++p) {
-#pragma unroll
-            for (int q = 0; q < XLD; ++q) {
-                const int f = threadIdx.x + q * NT;
-                const int ci = f / XPL;
-                Xs[p * XSZ + ci * XPP + (f - ci * XPL)] = xr[p][q];
-            }
-#pragma unroll
-            for (int q = 0; q < GLD; ++q) {
-                const int f = threadIdx.x + q * NT;
-                const int co = f / GPX;
-                Gs[p * GSZ + co * GPP + (f - co * GPX)] = gr[p][q];
-            }
-        }
+    auto fetch = [&](__amdgpu_buffer_rsrc_t rs, uint32_t v, uint32_t soff) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, v, soff, 0));
     };
 
     floatx16 acc[9];
+    auto clear = [&]() {
+#pragma unroll
+        for (int t = 0; t < 9; ++t)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) acc[t][q] = 0.f;
+    };
+    clear();
+
+    float xr[NX][8], gr[NG][8];
+    uint32_t xoff[NX], goff[NG];  // byte offset of a cell's first pixel in row 0
+    int xlim[NX], glim[NG];       // its pixels inside the row
+    auto strip = [&](int x0) {
+#pragma unroll
+        for (int i = 0; i < NX; ++i) {
+            const int e = threadIdx.x + NT * i, ci = e / (S + 2), s = e - ci * (S + 2);
+            const bool in = e < XC && c0 + ci < a.C;
+            xoff[i] = in ? (uint32_t)((c0 + ci) * xplane + x0 + s) * 4u : kPast;
+            xlim[i] = in ? (Wp - x0 - s + S - 1) / S : 0;
+        }
+#pragma unroll
+        for (int i = 0; i < NG; ++i) {
+            const int e = threadIdx.x + NT * i, co = e / S, s = e - co * S;
+            const bool in = e < GC && k0 + co < a.K;
+            goff[i] = in ? (uint32_t)((k0 + co) * gplane + x0 + s) * 4u : kPast;
+            glim[i] = in ? (a.W - x0 - s + S - 1) / S : 0;
+        }
+    };
+    auto load_x = [&](int i, int yy) {  // row yy of the padded image
+        const uint32_t soff = (uint32_t)(min(yy, Hp - 1) * Wp) * 4u;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) xr[i][j] = fetch(rx, j < xlim[i] ? xoff[i] + (uint32_t)(S * j * 4) : kPast, soff);
+    };
+    auto load_g = [&](int i, int y) {
+        const uint32_t soff = (uint32_t)(min(y, a.H - 1) * a.W) * 4u;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) gr[i][j] = fetch(rg, j < glim[i] ? goff[i] + (uint32_t)(S * j * 4) : kPast, soff);
+    };
+    u16x2 tiny = {0xffff, 0xffff};
+    auto store_x = [&](int i, int yy) {
+        const int e = threadIdx.x + NT * i, ci = e / (S + 2), s = e - ci * (S + 2);
+        u32x4 c[3];
+        split8(xr[i], c, tiny);
+        if (XC % NT == 0 || e < XC)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) xs[yy & 3][q * XPART + s * WGP + ci] = c[q];
+    };
+    auto store_g = [&](int i) {
+        const int e = threadIdx.x + NT * i, co = e / S, s = e - co * S;
+        u32x4 c[3];
+        split8(gr[i], c, tiny);
+        if (GC % NT == 0 || e < GC)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) gs[q * GPART + s * WGP + co] = c[q];
+    };
+
+    for (long r = lo; r < hi;) {
+        const WgRow w(a, r, 8 * S);
+        const long end = min(hi, r + (a.H - w.y));
+        image(w);
+        strip(w.x0);
+        // the strip's first rows; the row after them stays in registers
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+#pragma unroll
+            for (int i = 0; i < NX; ++i) load_x(i, w.y + k);
+#pragma unroll
+            for (int i = 0; i < NX; ++i) store_x(i, w.y + k);
+        }
+#pragma unroll
+        for (int i = 0; i < NG; ++i) load_g(i, w.y);
+#pragma unroll
+        for (int i = 0; i < NG; ++i) store_g(i);
+#pragma unroll
+        for (int i = 0; i < NX; ++i) load_x(i, w.y + 3);
+#pragma unroll
+        for (int i = 0; i < NG; ++i) load_g(i, w.y + 1);
+        __syncthreads();
+        for (int y = w.y; r < end; ++r, ++y) {
+            bf16x8 gf[S / 2][3], xf[2][3][3];
+#pragma unroll
+            for (int ks = 0; ks < S / 2; ++ks)
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+                    gf[ks][q] = __builtin_bit_cast(bf16x8, gs[q * GPART + (2 * ks + h) * WGP + 32 * wb + l32]);
+            auto frag = [&](int u, int buf) {  // u: ky S / 2 + ks
+                const int ky = u / (S / 2), ks = u % (S / 2);
+                const u32x4* row = xs[(y + ky) & 3];
+#pragma unroll
+                for (int kx = 0; kx < 3; ++kx)
+#pragma unroll
+                    for (int q = 0; q < 3; ++q)
+                        xf[buf][kx][q] = __builtin_bit_cast(bf16x8, row[q * XPART + (2 * ks + kx + h) * WGP + 32 * wa + l32]);
+            };
+            frag(0, 0);
+            __syncthreads();  // g's fragments are read: its next row may be stored
+            floatx16 sum[3];
+#pragma unroll
+            for (int u = 0; u < 3 * (S / 2); ++u) {
+                const int ky = u / (S / 2), ks = u % (S / 2), b = u & 1;
+                if (u + 1 < 3 * (S / 2)) frag(u + 1, b ^ 1);
+                if (ks == 0)
+#pragma unroll
+                    for (int kx = 0; kx < 3; ++kx)
+#pragma unroll
+                        for (int q = 0; q < 16; ++q) sum[kx][q] = 0.f;
+                __builtin_amdgcn_sched_barrier(0);
+                // a cell of the next row a group (the last stored row is never read)
+                if (u < NX) {
+                    store_x(u, y + 3);
+                    load_x(u, y + 4);
+                } else if (u - NX < NG) {
+                    store_g(u - NX);
+                    load_g(u - NX, y + 2);
+                }
+#pragma unroll
+                for (int x = 0; x < 6; ++x)
+#pragma unroll
+                    for (int kx = 0; kx < 3; ++kx) sum[kx] = mfma_bf16(xf[b][kx][kSplitA[x]], gf[ks][kSplitB[x]], sum[kx]);
+                if (ks == S / 2 - 1)
+#pragma unroll
+                    for (int kx = 0; kx < 3; ++kx)
+#pragma unroll
+                        for (int q = 0; q < 16; ++q) acc[3 * ky + kx][q] += sum[kx][q];
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            static_assert(NX + NG <= 3 * (S / 2), "staging groups");
+            __syncthreads();
+        }
+    }
+
+    float z = 0.f;  // NaN where a sum is not finite
 #pragma unroll
     for (int t = 0; t < 9; ++t)
 #pragma unroll
-        for (int q = 0; q < 16; ++q) acc[t][q] = 0.f;
-
-    // lane bases: patch channel 32 wa + l32, pixel + h;  g row 32 wb + l32, pixel + h
-    const int xb = (32 * wa + l32) * XPP + h;
-    const int gb = (32 * wb + l32) * GPP + h;
-    const int ntot = a.ntiles * a.npairs;
-    int tile = blockIdx.y;
-    if (tile < ntot) load(tile);
-    for (; tile < ntot; tile += gridDim.y) {
-        __syncthreads();
-        store();
-        __syncthreads();
-        if (tile + (int)gridDim.y < ntot) load(tile + gridDim.y);
-        // k steps s (pixel pairs 2s, 2s+1); step s+1's fragments are read during step s's MFMAs
-        constexpr int NSTEP = GPX / 2;
-        float gf[2][NPR], xf[2][NPR][9];
-        auto frag = [&](int st, int buf) {
-            const int py = (2 * st) / WTX, px = (2 * st) % WTX;
+        for (int q = 0; q < 16; ++q) z = __builtin_fmaf(acc[t][q], 0.f, z);
+    if (__syncthreads_or(z != 0.f || any_tiny(tiny))) {
+        clear();
+        const int c = c0 + 32 * wa + l32, k = k0 + 32 * wb + l32;
+        for (long r = lo; r < hi; ++r) {
+            const WgRow w(a, r, 8 * S);
+            image(w);
+            for (int px = 0; px < 8 * S; px += 2) {
+                const int x = w.x0 + px + h;
+                const float gv = fetch(rg, k < a.K && x < a.W ? (uint32_t)(k * gplane + x) * 4u : kPast, (uint32_t)(w.y * a.W) * 4u);
 #pragma unroll
-            for (int p = 0; p < NPR; ++p) {
-                gf[buf][p] = Gs[p * GSZ + gb + 2 * st];
-#pragma unroll
-                for (int t = 0; t < 9; ++t) xf[buf][p][t] = Xs[p * XSZ + xb + (py + t / 3) * XPX + px + t % 3];
+                for (int t = 0; t < 9; ++t) {
+                    const int xx = x + t % 3;
+                    const float xv = fetch(rx, c < a.C && xx < Wp ? (uint32_t)(c * xplane + xx) * 4u : kPast,
+                                           (uint32_t)((w.y + t / 3) * Wp) * 4u);
+                    acc[t] = mfma(xv, gv, acc[t]);
+                }
             }
-        };
-        frag(0, 0);
-#pragma unroll
-        for (int st = 0; st < NSTEP; ++st) {
-            const int b = st & 1;
-            if (st + 1 < NSTEP) frag(st + 1, b ^ 1);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int t = 0; t < 9; ++t)
-#pragma unroll
-                for (int p = 0; p < NPR; ++p) acc[t] = mfma(xf[b][p][t], gf[b][p], acc[t]);
-            __builtin_amdgcn_sched_barrier(0);
         }
     }
     // accumulator (t, q): c = 32 wa + 8 (q / 4) + 4 h + q % 4, co = 32 wb + l32 (slab-local)
@@ -857,20 +958,35 @@ hipError_t launch_tap(const TapArgs& a, const char* name, hipStream_t stream, un
     return hipGetLastError();
 }
 
-template <int NPR>
+// cells a k group of the weight gradient's strips (8 S columns): 64 columns, or 32 where that
+// leaves at least a sixth less of the columns empty.  Adjoint, 32 / 64 columns, us: W = 256
+// 848 / 819, 224 717 / 711, 160 495 / 501, 96 220 / 228, 28 87 / 91
+inline int wgrad_cells(int W) {
+    const int s = (W + 31) / 32;
+    return s % 2 && s <= 5 ? 4 : 8;
+}
+inline long wgrad_rows(const Dims& d) {
+    const int width = 8 * wgrad_cells(d.W);
+    return (long)((d.W + width - 1) / width) * d.H * d.N;
+}
+
+// wb += sum x0 g0 (+ sum x1 g1)
 int32_t weight_grad(const Dims& d, const float* x0, const float* g0, const float* x1, const float* g1, float* part,
                     int nsplit, float* wb, const char* name, hipStream_t stream) {
     WgArgs a{};
     a.x[0] = x0; a.g[0] = g0; a.x[1] = x1; a.g[1] = g1;
     a.N = d.N; a.C = d.C; a.K = d.K; a.H = d.H; a.W = d.W;
-    a.ntx = (d.W + WTX - 1) / WTX;
-    a.nty = (d.H + WTY - 1) / WTY;
-    a.ntiles = a.ntx * a.nty * d.N;
-    a.npairs = NPR == 1 && x1 ? 2 : 1;
+    const int cells = wgrad_cells(d.W);
+    a.ntx = (d.W + 8 * cells - 1) / (8 * cells);
+    a.nrows = wgrad_rows(d) * (x1 ? 2 : 1);
     a.part = part;
     const int ctn = d.Cpad / 64, ktn = d.Kpad / 64;
     dim3 grid(ctn * ktn, nsplit);
-    STADE_TIMED(name, stream, (wgrad_kernel<NPR><<<grid, NT, 0, stream>>>(a)));
+    if (cells == 8) {
+        STADE_TIMED(name, stream, (wgrad_kernel<8><<<grid, NT, 0, stream>>>(a)));
+    } else {
+        STADE_TIMED(name, stream, (wgrad_kernel<4><<<grid, NT, 0, stream>>>(a)));
+    }
     STADE_LAUNCHED("conv3x3 wgrad_kernel");
     const long nr = (long)ctn * ktn * 9 * 4096;
     STADE_TIMED("conv_wreduce", stream,
@@ -893,9 +1009,8 @@ int32_t run(const Ptrs& p, const Dims& d, hipStream_t stream) {
     const size_t nflag = up64((size_t)two * nprep);
     const size_t nout = up64((size_t)d.N * d.K * d.H * d.W);
     const int ctn = d.Cpad / 64, ktn = d.Kpad / 64;
-    const long ntiles = (long)((d.W + WTX - 1) / WTX) * ((d.H + WTY - 1) / WTY) * d.N;
     // ctn is 0 when C = 0 (no weight gradient to form)
-    const int nsplit = ctn == 0 ? 0 : (int)std::max(1L, std::min(ntiles, (long)std::max(1, 256 / (ctn * ktn))));
+    const int nsplit = ctn == 0 ? 0 : (int)std::max(1L, std::min(wgrad_rows(d), (long)std::max(1, 256 / (ctn * ktn))));
     const size_t npart = (MODE == TAN || d.C == 0) ? 0 : (size_t)nsplit * ctn * ktn * 9 * 4096;
     // the loss partials of the forward pass, where they do not fit the workspace's own
     const size_t nloss = 2 * (size_t)((d.W + tap_width(FWD_D) - 1) / tap_width(FWD_D)) * ((d.H + 3) / 4) * d.N * (d.Kpad / 64);
@@ -950,12 +1065,11 @@ int32_t run(const Ptrs& p, const Dims& d, hipStream_t stream) {
     }
     if (MODE == TAN || d.C == 0) return STADE_HIP_OK;
     // wb += sum xp g;  HVP: wbd += sum (xpd g + xp gd)
-    int32_t rc = weight_grad<1>(d, p.xp, G, nullptr, nullptr, part, nsplit, p.wb, "conv_wgrad", stream);
+    int32_t rc = weight_grad(d, p.xp, G, nullptr, nullptr, part, nsplit, p.wb, "conv_wgrad", stream);
     if (rc) return rc;
     if (MODE == HVP) {
-        // both products of wbd through the single-pair kernel, over twice the tiles (holding
-        // two pairs' tiles at once spilled registers and ran at 64 TFLOP/s)
-        rc = weight_grad<1>(d, p.xpd, G, p.xp, GD, part, nsplit, p.wbd, "conv_wgrad2", stream);
+        // both products of wbd in one launch over twice the rows
+        rc = weight_grad(d, p.xpd, G, p.xp, GD, part, nsplit, p.wbd, "conv_wgrad2", stream);
         if (rc) return rc;
     }
     // xpb interior += flipped taps over g;  HVP: xpbd += wd g + w gd

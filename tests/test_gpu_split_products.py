@@ -102,6 +102,17 @@ def test_split_conv_edges(mode, size):
     run_parity("conv3x3", mode, shapes, ints, precision="f32", scales={"w": s, "wd": s})
 
 
+@pytest.mark.parametrize("mode", ["b", "hv"])
+@pytest.mark.parametrize("size", [(1, 1, 1, 1, 1), (3, 5, 4, 50, 70), (2, 70, 66, 40, 63), (1, 3, 64, 300, 33), (2, 64, 3, 2, 129)])
+def test_split_conv_weight_gradient(mode, size):
+    """The weight gradient's strips of 32 and of 64 columns: one pixel, blocks whose rows cross
+    strips and images (more rows than blocks), two slabs each way, one past a strip's edge."""
+    shapes, ints = _conv(size)
+    s = 1.0 / np.sqrt(9.0 * size[1])
+    print(f"conv3x3_{mode} {size}", flush=True)
+    run_parity("conv3x3", mode, shapes, ints, precision="f32", scales={"w": s, "wd": s})
+
+
 @pytest.mark.parametrize("mode", ["b", "d", "hv"])
 @pytest.mark.parametrize("tiny", ["xp", "w"])
 def test_split_conv_tiny_operands(mode, tiny):
