@@ -106,6 +106,10 @@ __global__ __launch_bounds__(NT) void prep_kernel(const float* __restrict__ w, i
 // from the cache with four rows a block: 306 and 290; the splitting interleaved with the MFMAs
 // over a double-buffered patch: no faster.  Error against 64 bits 5.0e-7 -> 4.2e-7 (one source),
 // 3.0e-7 -> 1.8e-7 (two).
+// FRESH: fewer roundings at the total's size, for few channels, where v_mfma_f32_32x32x2_f32
+// would round less often than the six products of a tap and chunk do.  One source: a tap's
+// products are summed from zero and then added to the total.  Two sources (one chunk then): the
+// five small products of all taps first, then the h h of all taps, nine roundings in all.
 // A block that meets an element which the split cannot hold forms its tile again by
 // v_mfma_f32_32x32x2_f32 with operands straight from memory.
 // ------------------------------------------------------------------------------------------
@@ -138,7 +142,7 @@ struct TapArgs {
     double* partials;     // loss sums per block
 };
 
-template <int MODE, int TY>
+template <int MODE, int TY, bool FRESH>
 __global__ __launch_bounds__(64 * TY) void tap_kernel(TapArgs a) {
     constexpr int NP = tap_sources(MODE);  // sources = weight sets = outputs
     constexpr int TX = tap_width(MODE), NJ = TX / 32;
@@ -273,9 +277,12 @@ __global__ __launch_bounds__(64 * TY) void tap_kernel(TapArgs a) {
                 for (int j = 0; j < NJ; ++j)
                     pv[buf][p][j][q] = *reinterpret_cast<const bf16x8*>(lds + (p * 6 + 2 * q + h) * PLANE + ((wave + ky) * PXW + kx + 32 * j + l32) * 16);
     };
-    // two sources: the chunks' sums (acc) are added up here
-    floatx16 tot[NP == 2 ? NP : 1][2][NJ];
-    if constexpr (NP == 2) {
+    // two sources: the chunks' sums (acc) are added up here; one source, FRESH: the taps'
+    constexpr bool TOT = NP == 2 || FRESH;
+    // two sources, FRESH: the taps' small products first, then those of the h parts
+    constexpr int PASSES = NP == 2 && FRESH ? 2 : 1, STEPS = 9 * PASSES;
+    floatx16 tot[TOT ? NP : 1][2][NJ];
+    if constexpr (TOT) {
 #pragma unroll
         for (int o = 0; o < NP; ++o)
 #pragma unroll
@@ -295,15 +302,15 @@ __global__ __launch_bounds__(64 * TY) void tap_kernel(TapArgs a) {
         if (WLDS) read_weights(ch, 0, 0);
         read_pixels(0, 0);
         auto tap = [&](int t, int b) {
-            if (t < 8) {
-                read_pixels(t + 1, b ^ 1);
-                read_weights(ch, t + 1, b ^ 1);
+            if (t < STEPS - 1) {
+                read_pixels((t + 1) % 9, b ^ 1);
+                read_weights(ch, (t + 1) % 9, b ^ 1);
             } else if (!WLDS && ch + 1 < nchunks) {
                 read_weights(ch + 1, 0, b ^ 1);
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int x = 0; x < 6; ++x)
+            for (int x = t < 9 ? 0 : 5; x < (PASSES == 2 && t < 9 ? 5 : 6); ++x)
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -317,10 +324,10 @@ __global__ __launch_bounds__(64 * TY) void tap_kernel(TapArgs a) {
             __builtin_amdgcn_sched_barrier(0);
         };
 #pragma unroll
-        for (int t = 0; t < 9; ++t) {
+        for (int t = 0; t < STEPS; ++t) {
             tap(t, t & 1);
-            if constexpr (NP == 2) {
-                if (t != 8) continue;
+            if constexpr (TOT) {
+                if (!(NP == 1 && FRESH) && t != STEPS - 1) continue;
 #pragma unroll
                 for (int o = 0; o < NP; ++o)
 #pragma unroll
@@ -335,7 +342,7 @@ __global__ __launch_bounds__(64 * TY) void tap_kernel(TapArgs a) {
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if constexpr (!WLDS) {
+        if constexpr (!WLDS && STEPS % 2 == 1) {
             // (nine taps leave the next chunk's first weights in the other set: it is copied over)
 #pragma unroll
             for (int p = 0; p < NP; ++p)
@@ -346,7 +353,7 @@ __global__ __launch_bounds__(64 * TY) void tap_kernel(TapArgs a) {
         }
     }
 
-    if constexpr (NP == 2) {
+    if constexpr (TOT) {
 #pragma unroll
         for (int o = 0; o < NP; ++o)
 #pragma unroll
@@ -944,17 +951,23 @@ hipError_t launch_tap(const TapArgs& a, const char* name, hipStream_t stream, un
     // SIMD; the halo rows are a quarter of the patch instead of a half), otherwise four
     constexpr int TX = tap_width(MODE);
     const long tiles = (long)((a.W + TX - 1) / TX) * a.N * (a.Rpad / RT);
-    const bool tall = tap_sources(MODE) == 1 && tiles * ((a.H + 7) / 8) >= gemm::device_cus();
+    // (two sources: a chunk's sum is added to the total once)
+    const bool fresh = (a.Cin + 1) / 2 < 6 * (tap_sources(MODE) == 1 ? tap_chunks(a.Cin) : 1);
+    const bool tall = !fresh && tap_sources(MODE) == 1 && tiles * ((a.H + 7) / 8) >= gemm::device_cus();
     const int ty = tall ? 8 : 4;
     dim3 grid((a.W + TX - 1) / TX, (a.H + ty - 1) / ty, a.N * (a.Rpad / RT));
     nblocks = grid.x * grid.y * grid.z;
     if constexpr (tap_sources(MODE) == 1) {
         if (tall) {
-            STADE_TIMED(name, stream, (tap_kernel<MODE, 8><<<grid, 512, 0, stream>>>(a)));
+            STADE_TIMED(name, stream, (tap_kernel<MODE, 8, false><<<grid, 512, 0, stream>>>(a)));
             return hipGetLastError();
         }
     }
-    STADE_TIMED(name, stream, (tap_kernel<MODE, 4><<<grid, 256, 0, stream>>>(a)));
+    if (fresh) {
+        STADE_TIMED(name, stream, (tap_kernel<MODE, 4, true><<<grid, 256, 0, stream>>>(a)));
+    } else {
+        STADE_TIMED(name, stream, (tap_kernel<MODE, 4, false><<<grid, 256, 0, stream>>>(a)));
+    }
     return hipGetLastError();
 }
 

@@ -160,3 +160,24 @@ def test_split_conv_non_finite(value):
         ok = np.isfinite(want)
         if np.any(want[ok]):
             assert rel_err(got[ok], want[ok]) <= 1e-5, a
+
+
+@pytest.mark.parametrize("mode,outputs", [("b", ("out", "xpb")), ("d", ("out", "outd")), ("hv", ("out", "outd", "xpb", "xpbd"))])
+@pytest.mark.parametrize("size", [(1, 1, 2, 9, 40), (1, 3, 5, 17, 70), (2, 11, 9, 10, 33), (1, 10, 17, 12, 64)])
+def test_split_conv_few_channels(mode, outputs, size):
+    """Few channels, where the products are summed with fewer roundings: an element is a sum of
+    9 c products (the tangents 18 c) rounded at its size at most three times a tap, under
+    27 x 2^-24 of the terms' size (1.6e-6), and far less normwise; the seeds that xpb's terms
+    hold carry the error of out, its own and that of a product: 3 x 2^-24 more."""
+    shapes, ints = _conv(size)
+    s = 1.0 / np.sqrt(9.0 * size[1])
+    lib = oracle_lib("conv3x3", mode, "f64")
+    args = make_args(lib, f"conv3x3_{mode}", shapes, ints, {}, "split-conv-few", np.float32, None, {"w": s, "wd": s})
+    host = [v.astype(np.float64) if isinstance(v, np.ndarray) and v.dtype == np.float32 else v for _, _, v in args]
+    lib.call(f"conv3x3_{mode}", *host)
+    case = ParityCase("conv3x3", mode, args, (), "f32")
+    print(f"conv3x3_{mode} {size} few channels", flush=True)
+    case.run_gpu()
+    for (a, _, _), want, dev in zip(args, host, case.dev):
+        if a in outputs:
+            assert rel_err(to_host(dev).astype(np.float64), want) <= 1e-6, a
