@@ -13,10 +13,12 @@
 //   adjoint  g = outb + (0.5 (2 out)) lossb  (the accumulated outb, then reset to 0)
 //            wb[co][c][ky][kx] += sum_{n,y,x} g[n][co][y][x] xp[n][c][y+ky][x+kx]
 //            xpb[n][c][yp][xq] += sum_{co,ky,kx} w[co][c][ky][kx] g[n][co][yp-ky][xq-kx]
-// All three run on the matrix cores as implicit GEMMs by split bf16, with no im2col buffer: each
-// block stages its operands in LDS, and the taps read them there at shifted offsets.
-//   tap_kernel    forward (and the tangent's two products) and the interior of xpb, which
-//                 is the same shifted product on g with flipped, transposed weights
+// All three run on the matrix cores as implicit GEMMs, with no im2col buffer: each block stages
+// its operands in LDS, and the taps read them there at shifted offsets.  By split bf16, but for
+// the forward of the tangent and the HVP (fp32 MFMAs).
+//   tap_kernel    the adjoint's forward and the interior of xpb (and xpbd), which is the same
+//                 shifted product on g with flipped, transposed weights
+//   tap32_kernel  the forward of the tangent and the HVP: out and outd
 //   border_kernel the one-cell frame of xpb (taps that land on the zero padding): four 1-D
 //                 3-tap line correlations
 //   wgrad_kernel  split over pixel tiles, partial 9 x 64 x 64 weight gradients per block
@@ -52,7 +54,7 @@ __host__ __device__ __forceinline__ int tap_chunks(int Cin) { return (Cin + 15) 
 // ------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(NT) void prep_kernel(const float* __restrict__ w, int C, int K, u32x4* __restrict__ wf,
                                                   u32x4* __restrict__ wg, int* __restrict__ flags) {
-    const long nf = (long)tap_chunks(C) * 9 * 128 * ((K + 63) / 64), ng = wg ? (long)tap_chunks(K) * 9 * 128 * ((C + 63) / 64) : 0;
+    const long nf = wf ? (long)tap_chunks(C) * 9 * 128 * ((K + 63) / 64) : 0, ng = wg ? (long)tap_chunks(K) * 9 * 128 * ((C + 63) / 64) : 0;
     const long q = (long)blockIdx.x * NT + threadIdx.x;
     u16x2 tiny = {0xffff, 0xffff};
     if (q < nf + ng) {
@@ -96,10 +98,9 @@ __global__ __launch_bounds__(NT) void prep_kernel(const float* __restrict__ w, i
 // from the cache beside the MFMAs instead, a tap's weights wait for every older load of the
 // wave, the next chunk's pixels from HBM among them (loads return in order).  Eight rows give
 // two waves a SIMD.
-// Two sources (NP = 2; tangent, HVP: four products a tap into two outputs): NJ = 1, the weights
-// (two sets, too many for LDS) from the cache.  The two outputs' sums are kept per chunk and then
-// added to their totals, which more than halves their rounding (a tangent's loss sums products
-// of both that cancel).
+// Two sources (NP = 2; the HVP's xpb and xpbd: three products a tap into two outputs): NJ = 1, the
+// weights (two sets, too many for LDS) from the cache.  The two outputs' sums are kept per chunk
+// and then added to their totals, which more than halves their rounding.
 // Measured, us with fp32 MFMAs -> split: 8 x 64 -> 64 x 256^2, forward 391 -> 287, xpb 385 -> 270;
 // the matrix cores are busy for 40 % of it.  Without the MFMAs' operands being staged, the
 // MFMAs and the epilogue alone take 186 and 157 us (672 and 406 MB of HBM traffic); weights
@@ -117,11 +118,13 @@ constexpr int RT = 64, CC = 16;
 constexpr int WCELLS = 9 * 6 * 64;   // weight cells of a chunk and row tile
 enum { FWD_B, FWD_D, FWD_HV, DG_B, DG_HV };
 constexpr int tap_sources(int mode) { return mode == FWD_B || mode == DG_B ? 1 : 2; }
-constexpr int tap_width(int mode) { return tap_sources(mode) == 1 ? 64 : 32; }
+constexpr bool tap_split(int mode) { return mode != FWD_D && mode != FWD_HV; }
+constexpr int tap_width(int mode) { return mode == DG_HV ? 32 : 64; }
 
 struct TapArgs {
     const float* src[2];   // sources (n, cin, SH, SW)
     const u32x4* wt[2];    // split weights (prep_kernel)
+    const float* wt32[2];  // the tangent's forward: weights [cin][9][Rpad] (prep32_kernel)
     const float* w[2];     // the weights themselves: (r, cin, t) at w[r * wr + cin * wc + (flip ? 8 - t : t)]
     long wr, wc;
     bool flip;
@@ -142,6 +145,83 @@ struct TapArgs {
     double* partials;     // loss sums per block
 };
 
+// The outputs of a wave's tile: pixel row y, columns x0..., rows of tile rt.
+template <int MODE, int NJ>
+__device__ __forceinline__ void tap_epilogue(const TapArgs& a, floatx16 (&acc)[tap_sources(MODE)][2][NJ], int n, int rt, int x0, int y,
+                                             double* red) {
+    constexpr bool FWD = MODE == FWD_B || MODE == FWD_D || MODE == FWD_HV;
+    constexpr int NV = MODE == FWD_B ? 1 : 2;
+    const int h = (threadIdx.x & 63) >> 5, l32 = threadIdx.x & 31;
+    // accumulator (i, j, q) is row r = rt*64 + 32 i + 8 (q / 4) + 4 h + q % 4,
+    // pixel x = x0 + 32 j + l32 of row y
+    double ls[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) ls[k] = 0.0;
+    float lb = 0.f, lbd = 0.f;
+    if constexpr (MODE == FWD_B || MODE == FWD_HV) lb = a.lossb[0];
+    if constexpr (MODE == FWD_HV) lbd = a.lossbd[0];
+    // The read-modify-write inputs (outb, outbd of the forward adjoint; xpb, xpbd of the
+    // interior) are all loaded before any store: the output arrays may alias as far as the
+    // compiler knows, so interleaving would serialise one HBM round trip per element.
+    constexpr bool RMW = MODE != FWD_D;
+    constexpr int NR = (MODE == FWD_HV || MODE == DG_HV) ? 2 : 1;
+    float pre[NR][2][NJ][16];
+    auto index = [&](int i, int j, int q, long& oi) {
+        const int x = x0 + 32 * j + l32;
+        const int r = rt * RT + 32 * i + 8 * (q >> 2) + 4 * h + (q & 3);
+        oi = ((long)(n * a.R + r) * a.OH + y + a.oofs) * a.OW + x + a.oofs;
+        return y < a.H && x < a.W && r < a.R;
+    };
+    if constexpr (RMW) {
+        const float* s0 = FWD ? a.ob : a.o0;
+        const float* s1 = FWD ? a.obd : a.o1;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int q = 0; q < 16; ++q) {
+                    long oi;
+                    const bool ok = index(i, j, q, oi);
+                    pre[0][i][j][q] = ok ? s0[oi] : 0.f;
+                    if constexpr (NR == 2) pre[NR - 1][i][j][q] = ok ? s1[oi] : 0.f;
+                }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                long oi;
+                if (!index(i, j, q, oi)) continue;
+                const float v = acc[0][i][j][q];
+                if constexpr (FWD) {
+                    a.o0[oi] = v;
+                    ls[0] += 0.5 * (double)v * (double)v;
+                    if constexpr (MODE == FWD_B) {
+                        a.g0[oi] = pre[0][i][j][q] + (0.5f * (2.0f * v)) * lb;
+                        a.ob[oi] = 0.f;
+                    } else {
+                        const float vd = acc[1][i][j][q];
+                        a.o1[oi] = vd;
+                        ls[1] += 0.5 * ((double)(2.0f * v) * (double)vd);
+                        if constexpr (MODE == FWD_HV) {
+                            const float c8 = 0.5f * (2.0f * v);
+                            a.g1[oi] = pre[NR - 1][i][j][q] + (lb * (0.5f * (2.0f * vd)) + c8 * lbd);
+                            a.g0[oi] = pre[0][i][j][q] + c8 * lb;
+                            a.ob[oi] = 0.f;
+                            a.obd[oi] = 0.f;
+                        }
+                    }
+                } else {
+                    a.o0[oi] = pre[0][i][j][q] + v;
+                    if constexpr (MODE == DG_HV) a.o1[oi] = pre[NR - 1][i][j][q] + acc[1][i][j][q];
+                }
+            }
+    if constexpr (FWD) block_partials<NV>(ls, red, a.partials);
+}
+
 template <int MODE, int TY, bool FRESH>
 __global__ __launch_bounds__(64 * TY) void tap_kernel(TapArgs a) {
     constexpr int NP = tap_sources(MODE);  // sources = weight sets = outputs
@@ -150,12 +230,10 @@ __global__ __launch_bounds__(64 * TY) void tap_kernel(TapArgs a) {
     constexpr int PLANE = PPL * 16;                                // bytes of one (part, octet) plane
     constexpr bool WLDS = NP == 1;                                 // weights staged in LDS
     constexpr int WPT = WLDS ? (WCELLS + NTH - 1) / NTH : 1;       // weight cells of a thread
-    constexpr bool FWD = MODE == FWD_B || MODE == FWD_D || MODE == FWD_HV;
-    constexpr int NV = MODE == FWD_B ? 1 : 2;
 
     __shared__ __attribute__((aligned(16))) char lds[NP * 6 * PLANE];
     __shared__ u32x4 wlds[WLDS ? WCELLS : 1];
-    __shared__ double red[16 * NV];
+    __shared__ double red[16];
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, l32 = lane & 31;
@@ -409,75 +487,192 @@ __global__ __launch_bounds__(64 * TY) void tap_kernel(TapArgs a) {
         }
     }
 
-    // epilogue: accumulator (i, j, q) is row r = rt*64 + 32 i + 8 (q / 4) + 4 h + q % 4,
-    // pixel x = x0 + 32 j + l32 of row y = y0 + wave
-    double ls[NV];
+    tap_epilogue<MODE, NJ>(a, acc, n, rt, x0, y0 + wave, red);
+}
+
+// ------------------------------------------------------------------------------------------
+// the tangent's forward (tangent, HVP): out and outd by fp32 MFMAs (v_mfma_f32_32x32x2_f32).
+// lossd is a sum of products of out and outd that cancel: its relative error is theirs times a
+// condition number that is 10 for one set of inputs and 100 for another, so that two forms of
+// rounding agree in lossd to 5e-6 or not by chance.  By split bf16 this kernel takes 0.66 of the
+// time (8 x 64 -> 64 x 256^2: 1028 -> 678 us a tangent), with half the error in out and outd, but
+// with a lossd that differs by up to 6e-6 (4 x 32 -> 48 x 112 x 100) from that of a sum rounded in
+// channel order.
+//
+// Block: 256 threads, a 64-row (r) x (64 x 4 pixel) output tile.  Wave w owns pixel row
+// y0 + w: 2 x 2 MFMA 32 x 32 tiles (r halves x pixel halves) of each output.  Input channels
+// advance 8 at a time; each step stages the (4+2) x (64+2) patch of every channel and the 9 x 64
+// weight rows in LDS.  The next step's global loads are issued into registers before the MFMAs
+// of the current one.  The MFMA k pair (lane / 32) is a pair of channels at the same tap, so
+// every LDS read has a lane base plus an immediate offset.  72 % of the fp32 matrix peak
+// (8 x 64 -> 64 x 256^2).
+// ------------------------------------------------------------------------------------------
+// its weights and their directions: wt[cin][t][r], rows padded to a multiple of 64 with zeros
+__global__ __launch_bounds__(NT) void prep32_kernel(const float* __restrict__ w, const float* __restrict__ wd, int C, int K,
+                                                    float* __restrict__ wf, float* __restrict__ wfd, int Kpad) {
+    const long q = (long)blockIdx.x * NT + threadIdx.x;
+    if (q >= (long)C * 9 * Kpad) return;
+    const int r = (int)(q % Kpad);
+    const long ct = q / Kpad;
+    const int t = (int)(ct % 9), c = (int)(ct / 9);
+    const long i = ((long)r * C + c) * 9 + t;
+    wf[q] = r < K ? w[i] : 0.f;
+    wfd[q] = r < K ? wd[i] : 0.f;
+}
+
+template <int MODE>
+__global__ __launch_bounds__(NT) void tap32_kernel(TapArgs a) {
+    constexpr int NP = 2;  // sources = weight sets = outputs
+    constexpr int TX = 64, TY = 4, CC = 8;
+    constexpr int PXW = TX + 2, PYH = TY + 2, PPL = PXW * PYH;  // patch row, rows, plane (floats)
+    constexpr int KW = 9 * RT;                                    // weight floats per channel
+    constexpr int PSZ = CC * PPL, WSZ = CC * KW;
+    constexpr int WLD = NP * WSZ / 4 / NT;
+    static_assert(NP * WSZ % (4 * NT) == 0, "weight stage");
+
+    __shared__ float lds[NP * (PSZ + WSZ)];
+    __shared__ double red[32];
+    float* Ps = lds;
+    float* Ws = lds + NP * PSZ;
+
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int h = lane >> 5, l32 = lane & 31;
+    const int x0 = blockIdx.x * TX, y0 = blockIdx.y * TY;
+    const int rtiles = a.Rpad / RT;
+    const int n = blockIdx.z / rtiles, rt = blockIdx.z - n * rtiles;
+
+    // Patch staging by rows: the NP * CC * PYH = 96 patch rows of PXW = 66 floats; wave w
+    // takes rows w, w + 4, ..., one column per lane (columns 0..63), so the channel, row and
+    // row bounds are wave-uniform (scalar) and a lane's address is a row base plus its lane;
+    // columns 64, 65 of every row go to threads 0..191, one element each.
+    constexpr int PROWS = NP * CC * PYH, RPW = PROWS / 4;
+    static_assert(PROWS % 4 == 0 && PXW == 66 && 2 * PROWS <= NT, "patch rows");
+    float pr[RPW + 1];
+    float4 wr[WLD];
+    // Staging loads are buffer loads: a scalar resource per source image n (and per weight
+    // set), the row part of a patch address as a scalar offset (patch rows are wave-uniform)
+    // and the column as the lane's offset.  An element outside the source reads offset =
+    // the resource's size, which returns 0.  Vector registers hold no 64-bit addresses, so the
+    // staging fits two waves per SIMD without spilling.  (The host keeps one image of a
+    // source and a weight set under 2^31 bytes.)
+    const long plane = (long)a.SH * a.SW;
+    const uint32_t sbytes = (uint32_t)((long)a.Cin * plane * 4);
+    const uint32_t wbytes = (uint32_t)((long)a.Cin * 9 * a.Rpad * 4);
+    __amdgpu_buffer_rsrc_t rs[NP], rw[NP];
 #pragma unroll
-    for (int k = 0; k < NV; ++k) ls[k] = 0.0;
-    float lb = 0.f, lbd = 0.f;
-    if constexpr (MODE == FWD_B || MODE == FWD_HV) lb = a.lossb[0];
-    if constexpr (MODE == FWD_HV) lbd = a.lossbd[0];
-    const int y = y0 + wave;
-    // The read-modify-write inputs (outb, outbd of the forward adjoint; xpb, xpbd of the
-    // interior) are all loaded before any store: the output arrays may alias as far as the
-    // compiler knows, so interleaving would serialise one HBM round trip per element.
-    constexpr bool RMW = MODE != FWD_D;
-    constexpr int NR = (MODE == FWD_HV || MODE == DG_HV) ? 2 : 1;
-    float pre[NR][2][NJ][16];
-    auto index = [&](int i, int j, int q, long& oi) {
-        const int x = x0 + 32 * j + l32;
-        const int r = rt * RT + 32 * i + 8 * (q >> 2) + 4 * h + (q & 3);
-        oi = ((long)(n * a.R + r) * a.OH + y + a.oofs) * a.OW + x + a.oofs;
-        return y < a.H && x < a.W && r < a.R;
+    for (int p = 0; p < NP; ++p) {
+        rs[p] = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.src[p] + (long)n * a.Cin * plane), (short)0, sbytes,
+                                                  kBufWord3);
+        rw[p] = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.wt32[p] + rt * RT), (short)0, wbytes, kBufWord3);
+    }
+    const int sx_l = x0 + lane + a.ofs;
+    const uint32_t lane_col = (unsigned)sx_l < (unsigned)a.SW ? (uint32_t)sx_l * 4u : sbytes;
+    auto load = [&](int c0) {
+#pragma unroll
+        for (int i = 0; i < RPW; ++i) {
+            const int rr = wave + 4 * i;  // wave-uniform patch row (p, cc, ty)
+            const int p = rr / (CC * PYH);
+            const int rem = rr - p * (CC * PYH);
+            const int cc = rem / PYH, ty = rem - cc * PYH;
+            const int c = c0 + cc, sy = y0 + ty + a.ofs;
+            const bool ok = c < a.Cin && (unsigned)sy < (unsigned)a.SH;
+            const uint32_t soff = ok ? (uint32_t)(((long)c * a.SH + sy) * a.SW * 4) : 0u;
+            const uint32_t voff = ok ? lane_col : sbytes;
+            pr[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(p ? rs[NP - 1] : rs[0], voff, soff, 0));
+        }
+        if (threadIdx.x < 2 * PROWS) {
+            // columns 64, 65: the row varies across a wave, so the whole offset is the lane's
+            const int rr = threadIdx.x >> 1, col = 64 + (threadIdx.x & 1);
+            const int p = rr / (CC * PYH);
+            const int rem = rr - p * (CC * PYH);
+            const int cc = rem / PYH, ty = rem - cc * PYH;
+            const int c = c0 + cc, sy = y0 + ty + a.ofs, sx = x0 + col + a.ofs;
+            float v = 0.f;
+            if (c < a.Cin && (unsigned)sy < (unsigned)a.SH && (unsigned)sx < (unsigned)a.SW)
+                v = a.src[p][((long)(n * a.Cin + c) * a.SH + sy) * a.SW + sx];
+            pr[RPW] = v;
+        }
+        const uint32_t wsoff = (uint32_t)((long)c0 * 9 * a.Rpad * 4);
+#pragma unroll
+        for (int q = 0; q < WLD; ++q) {
+            const int f = threadIdx.x + q * NT;  // float4 slot of [w][cc][t][r]
+            const int wi = __builtin_amdgcn_readfirstlane(f / (WSZ / 4));  // uniform per wave
+            const int rem = f - wi * (WSZ / 4);
+            const int row = rem / (RT / 4), r4 = (rem - row * (RT / 4)) * 4;
+            const int cc = row / 9, t = row - cc * 9;
+            const uint32_t voff = c0 + cc < a.Cin ? (uint32_t)(((cc * 9 + t) * a.Rpad + r4) * 4) : wbytes;
+            const v4f x = __builtin_amdgcn_raw_buffer_load_b128(wi ? rw[NP - 1] : rw[0], voff, wsoff, 0);
+            wr[q] = make_float4(x.x, x.y, x.z, x.w);
+        }
     };
-    if constexpr (RMW) {
-        const float* s0 = FWD ? a.ob : a.o0;
-        const float* s1 = FWD ? a.obd : a.o1;
+    auto store = [&]() {
+        // patch row rr = (p, cc, ty) is at Ps + p * PSZ + cc * PPL + ty * PXW = Ps + rr * PXW
+#pragma unroll
+        for (int i = 0; i < RPW; ++i) Ps[(wave + 4 * i) * PXW + lane] = pr[i];
+        if (threadIdx.x < 2 * PROWS) Ps[(threadIdx.x >> 1) * PXW + 64 + (threadIdx.x & 1)] = pr[RPW];
+#pragma unroll
+        for (int q = 0; q < WLD; ++q) {
+            const int f = threadIdx.x + q * NT;
+            *reinterpret_cast<float4*>(Ws + 4 * f) = wr[q];
+        }
+    };
+
+    floatx16 acc[NP][2][2];
+#pragma unroll
+    for (int o = 0; o < NP; ++o)
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int j = 0; j < NJ; ++j)
+            for (int j = 0; j < 2; ++j)
 #pragma unroll
-                for (int q = 0; q < 16; ++q) {
-                    long oi;
-                    const bool ok = index(i, j, q, oi);
-                    pre[0][i][j][q] = ok ? s0[oi] : 0.f;
-                    if constexpr (NR == 2) pre[NR - 1][i][j][q] = ok ? s1[oi] : 0.f;
+                for (int q = 0; q < 16; ++q) acc[o][i][j][q] = 0.f;
+
+    // lane bases: patch channel (2 qq + h), row (wave + ky), column (32 j + l32 + kx);
+    // weight row (2 qq + h, t), column 32 i + l32
+    const int pbase = h * PPL + wave * PXW + l32;
+    const int wbase = h * KW + l32;
+    const int nchunks = (a.Cin + CC - 1) / CC;
+    if (nchunks > 0) load(0);
+    for (int ch = 0; ch < nchunks; ++ch) {
+        __syncthreads();
+        store();
+        __syncthreads();
+        if (ch + 1 < nchunks) load((ch + 1) * CC);
+        // k steps st = (channel pair qq, tap t); the fragments of step st+1 are read from LDS
+        // while the MFMAs of step st run (two register sets; the scheduling barriers keep
+        // the compiler from sinking each read to its use)
+        constexpr int NSTEP = CC / 2 * 9;
+        float pf[2][NP][2], wf[2][NP][2];
+        auto frag = [&](int st, int buf) {
+            const int qq = st / 9, t = st % 9, ky = t / 3, kx = t % 3;
+#pragma unroll
+            for (int p = 0; p < NP; ++p)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) pf[buf][p][j] = Ps[p * PSZ + pbase + 2 * qq * PPL + ky * PXW + kx + 32 * j];
+#pragma unroll
+            for (int p = 0; p < NP; ++p)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) wf[buf][p][i] = Ws[p * WSZ + wbase + (2 * qq * 9 + t) * RT + 32 * i];
+        };
+        frag(0, 0);
+#pragma unroll
+        for (int st = 0; st < NSTEP; ++st) {
+            const int b = st & 1;
+            if (st + 1 < NSTEP) frag(st + 1, b ^ 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    acc[0][i][j] = mfma(wf[b][0][i], pf[b][0][j], acc[0][i][j]);
+                    acc[1][i][j] = mfma(wf[b][1][i], pf[b][0][j], acc[1][i][j]);
+                    acc[1][i][j] = mfma(wf[b][0][i], pf[b][1][j], acc[1][i][j]);
                 }
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j)
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                long oi;
-                if (!index(i, j, q, oi)) continue;
-                const float v = acc[0][i][j][q];
-                if constexpr (FWD) {
-                    a.o0[oi] = v;
-                    ls[0] += 0.5 * (double)v * (double)v;
-                    if constexpr (MODE == FWD_B) {
-                        a.g0[oi] = pre[0][i][j][q] + (0.5f * (2.0f * v)) * lb;
-                        a.ob[oi] = 0.f;
-                    } else {
-                        const float vd = acc[1][i][j][q];
-                        a.o1[oi] = vd;
-                        ls[1] += 0.5 * ((double)(2.0f * v) * (double)vd);
-                        if constexpr (MODE == FWD_HV) {
-                            const float c8 = 0.5f * (2.0f * v);
-                            a.g1[oi] = pre[NR - 1][i][j][q] + (lb * (0.5f * (2.0f * vd)) + c8 * lbd);
-                            a.g0[oi] = pre[0][i][j][q] + c8 * lb;
-                            a.ob[oi] = 0.f;
-                            a.obd[oi] = 0.f;
-                        }
-                    }
-                } else {
-                    a.o0[oi] = pre[0][i][j][q] + v;
-                    if constexpr (MODE == DG_HV) a.o1[oi] = pre[NR - 1][i][j][q] + acc[1][i][j][q];
-                }
-            }
-    if constexpr (FWD) block_partials<NV>(ls, red, a.partials);
+
+    tap_epilogue<MODE, 2>(a, acc, n, rt, x0, y0 + wave, red);
 }
 
 // loss (and lossd) += the sum of the tap kernel's block partials, rounded once to Float32
@@ -947,26 +1142,24 @@ inline size_t up64(size_t n) { return (n + 63) / 64 * 64; }
 
 template <int MODE>
 hipError_t launch_tap(const TapArgs& a, const char* name, hipStream_t stream, unsigned& nblocks) {
+    constexpr int TX = tap_width(MODE), NP = tap_sources(MODE);
     // one source: eight pixel rows a block where that still gives every CU one (two waves a
     // SIMD; the halo rows are a quarter of the patch instead of a half), otherwise four
-    constexpr int TX = tap_width(MODE);
     const long tiles = (long)((a.W + TX - 1) / TX) * a.N * (a.Rpad / RT);
     // (two sources: a chunk's sum is added to the total once)
-    const bool fresh = (a.Cin + 1) / 2 < 6 * (tap_sources(MODE) == 1 ? tap_chunks(a.Cin) : 1);
-    const bool tall = !fresh && tap_sources(MODE) == 1 && tiles * ((a.H + 7) / 8) >= gemm::device_cus();
+    const bool fresh = (a.Cin + 1) / 2 < 6 * (NP == 1 ? tap_chunks(a.Cin) : 1);
+    const bool tall = NP == 1 && !fresh && tiles * ((a.H + 7) / 8) >= gemm::device_cus();
     const int ty = tall ? 8 : 4;
-    dim3 grid((a.W + TX - 1) / TX, (a.H + ty - 1) / ty, a.N * (a.Rpad / RT));
+    const dim3 grid((a.W + TX - 1) / TX, (a.H + ty - 1) / ty, a.N * (a.Rpad / RT));
     nblocks = grid.x * grid.y * grid.z;
-    if constexpr (tap_sources(MODE) == 1) {
-        if (tall) {
-            STADE_TIMED(name, stream, (tap_kernel<MODE, 8, false><<<grid, 512, 0, stream>>>(a)));
-            return hipGetLastError();
-        }
-    }
-    if (fresh) {
+    if constexpr (!tap_split(MODE)) {
+        STADE_TIMED(name, stream, (tap32_kernel<MODE><<<grid, NT, 0, stream>>>(a)));
+    } else if (fresh) {
         STADE_TIMED(name, stream, (tap_kernel<MODE, 4, true><<<grid, 256, 0, stream>>>(a)));
-    } else {
+    } else if (!tall) {
         STADE_TIMED(name, stream, (tap_kernel<MODE, 4, false><<<grid, 256, 0, stream>>>(a)));
+    } else if constexpr (NP == 1) {
+        STADE_TIMED(name, stream, (tap_kernel<MODE, 8, false><<<grid, 512, 0, stream>>>(a)));
     }
     return hipGetLastError();
 }
@@ -1014,10 +1207,13 @@ int32_t run(const Ptrs& p, const Dims& d, hipStream_t stream) {
     WsCall call_(stream);
     Workspace* ws = call_.ws;
     if (!ws) return STADE_HIP_ENOMEM;
-    // split weights: 16-byte cells, 3 parts of 128 a tap, chunk and row tile (in floats below)
-    const size_t cf = (size_t)tap_chunks(d.C) * 9 * 128 * (d.Kpad / 64), cg = (size_t)tap_chunks(d.K) * 9 * 128 * (d.Cpad / 64);
-    const size_t nwf = cf * 12, nwg = cg * 12;
-    const int nprep = (int)((cf + (MODE == TAN ? 0 : cg) + NT - 1) / NT);
+    // split weights (the adjoint's forward; xpb): 16-byte cells, 3 parts of 128 a tap, chunk and
+    // row tile (in floats below).  The tangent's forward: both weight sets in fp32
+    const size_t cf = MODE == ADJ ? (size_t)tap_chunks(d.C) * 9 * 128 * (d.Kpad / 64) : 0;
+    const size_t cg = MODE == TAN ? 0 : (size_t)tap_chunks(d.K) * 9 * 128 * (d.Cpad / 64);
+    const size_t n32 = MODE == ADJ ? 0 : up64((size_t)d.C * 9 * d.Kpad);
+    const size_t nwf = cf * 12 + 2 * n32, nwg = cg * 12;
+    const int nprep = (int)((cf + cg + NT - 1) / NT);
     const int two = MODE == ADJ ? 1 : 2;
     const size_t nflag = up64((size_t)two * nprep);
     const size_t nout = up64((size_t)d.N * d.K * d.H * d.W);
@@ -1025,34 +1221,32 @@ int32_t run(const Ptrs& p, const Dims& d, hipStream_t stream) {
     // ctn is 0 when C = 0 (no weight gradient to form)
     const int nsplit = ctn == 0 ? 0 : (int)std::max(1L, std::min(wgrad_rows(d), (long)std::max(1, 256 / (ctn * ktn))));
     const size_t npart = (MODE == TAN || d.C == 0) ? 0 : (size_t)nsplit * ctn * ktn * 9 * 4096;
-    // the loss partials of the forward pass, where they do not fit the workspace's own
-    const size_t nloss = 2 * (size_t)((d.W + tap_width(FWD_D) - 1) / tap_width(FWD_D)) * ((d.H + 3) / 4) * d.N * (d.Kpad / 64);
-    const bool own_loss = MODE != ADJ && nloss > (size_t)kPartialSlots;
-    const size_t total = two * nwf + (MODE == TAN ? 0 : two * nwg + two * nout) + nflag + up64(npart) + (own_loss ? 2 * nloss : 0);
+    const size_t total = nwf + (MODE == TAN ? 0 : two * nwg + two * nout) + nflag + npart;
     float* base = (float*)scratch(sizeof(float) * total + 256);
     if (!base) return scratch_error();
-    float* wf0 = base;
-    float* wf1 = wf0 + nwf;
-    float* wg0 = wf0 + two * nwf;
+    float* wf = base;
+    float* wg0 = wf + nwf;
     float* wg1 = wg0 + nwg;
     float* G = wg0 + (MODE == TAN ? 0 : two * nwg);
     float* GD = G + nout;
     int* flags = (int*)(G + (MODE == TAN ? 0 : two * nout));
     float* part = (float*)(flags + nflag);
-    double* const lpart = own_loss ? (double*)(part + up64(npart)) : ws->partials;
 
-    // weights in the tap kernel's form
+    // weights in the tap kernels' forms
+    if (n32 > 0) {
+        STADE_TIMED("conv_prep", stream, (prep32_kernel<<<(unsigned)((n32 + NT - 1) / NT), NT, 0, stream>>>(p.w, p.wd, d.C, d.K, wf, wf + n32, d.Kpad)));
+        STADE_LAUNCHED("conv3x3 prep32_kernel");
+    }
     for (int s = 0; s < two && nprep > 0; ++s) {
-        STADE_TIMED("conv_prep", stream, (prep_kernel<<<nprep, NT, 0, stream>>>(s ? p.wd : p.w, d.C, d.K, (u32x4*)(s ? wf1 : wf0),
-                                                                               MODE == TAN ? nullptr : (u32x4*)(s ? wg1 : wg0),
-                                                                               flags + s * nprep)));
+        STADE_TIMED("conv_prep", stream, (prep_kernel<<<nprep, NT, 0, stream>>>(s ? p.wd : p.w, d.C, d.K, MODE == ADJ ? (u32x4*)wf : nullptr,
+                                                                               (u32x4*)(s ? wg1 : wg0), flags + s * nprep)));
         STADE_LAUNCHED("conv3x3 prep_kernel");
     }
     // forward: out (and outd), loss (and lossd); adjoint seeds g (and gd), outb (and outbd) reset
     {
         TapArgs a{};
         a.src[0] = p.xp; a.src[1] = p.xpd;
-        a.wt[0] = (u32x4*)wf0; a.wt[1] = (u32x4*)wf1;
+        a.wt[0] = (u32x4*)wf; a.wt32[0] = wf; a.wt32[1] = wf + n32;
         a.w[0] = p.w; a.w[1] = p.wd; a.wr = 9L * d.C; a.wc = 9; a.flip = false;
         a.flags = flags; a.nflags = two * nprep;
         a.Cin = d.C; a.R = d.K; a.Rpad = d.Kpad; a.N = d.N;
@@ -1062,7 +1256,7 @@ int32_t run(const Ptrs& p, const Dims& d, hipStream_t stream) {
         a.OH = d.H; a.OW = d.W; a.oofs = 0;
         a.g0 = G; a.g1 = GD; a.ob = p.outb; a.obd = p.outbd;
         a.lossb = p.lossb; a.lossbd = p.lossbd;
-        a.partials = lpart;
+        a.partials = ws->partials;
         unsigned nblocks = 0;
         hipError_t e;
         if (MODE == ADJ) e = launch_tap<FWD_B>(a, "conv_fwd", stream, nblocks);
@@ -1070,9 +1264,9 @@ int32_t run(const Ptrs& p, const Dims& d, hipStream_t stream) {
         else e = launch_tap<FWD_HV>(a, "conv_fwd_hv", stream, nblocks);
         if (e != hipSuccess) return check_hip(e, "conv3x3 tap_kernel (forward)");
         if (MODE == ADJ) {
-            STADE_TIMED("conv_loss", stream, (loss_kernel<1><<<1, NT, 0, stream>>>(lpart, (int)nblocks, p.loss, nullptr)));
+            STADE_TIMED("conv_loss", stream, (loss_kernel<1><<<1, NT, 0, stream>>>(ws->partials, (int)nblocks, p.loss, nullptr)));
         } else {
-            STADE_TIMED("conv_loss", stream, (loss_kernel<2><<<1, NT, 0, stream>>>(lpart, (int)nblocks, p.loss, p.lossd)));
+            STADE_TIMED("conv_loss", stream, (loss_kernel<2><<<1, NT, 0, stream>>>(ws->partials, (int)nblocks, p.loss, p.lossd)));
         }
         STADE_LAUNCHED("conv3x3 loss_kernel");
     }
