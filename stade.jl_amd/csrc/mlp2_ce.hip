@@ -8,8 +8,13 @@
 // same-address fp32 atomics per weight; the reference's tiled contraction twins
 // (`cgen_adjoint_contraction_` 14762) are CUDA-only.
 //
-// Here the three contractions run on the fp32 matrix cores (gemm_f32.hpp), each with its
-// elementwise neighbours fused into the epilogue:
+// Here the three contractions run on the matrix cores, each with its elementwise neighbours fused
+// into the epilogue: the forward by fp32 MFMAs (gemm_f32.hpp), the backward pair by split bf16
+// (gemm_split.hpp).  By split bf16 the adjoint's forward takes as long (4096 x 784 -> 1024: 70 us) and
+// the tangent's dual one less (179 -> 121 us), but the sums over the batch that follow are then
+// further from 64 bits (b2b at 1000 x 500 x 700 3.1e-8 -> 5.8e-8, w2b 7.2e-8 -> 9.0e-8, b1b 6.0e-8 ->
+// 7.6e-8, rms over 30 seeds), and lossd, whose terms cancel, moves by more than 5e-6 in 1 of 30
+// draws:
 //   S1 = W1 X            epilogue h1 = tanh(S1 + b1)                 (H x B, K = I)
 //   head (per sample)    z = W2 h1 + b2, CE, d2 = dloss/dz, zb reset,
 //                        d1 = (1 - h1^2) (h1b + W2' d2), h1b reset    (one wave per sample)
@@ -22,7 +27,7 @@
 #include "internal.hpp"
 
 #include <algorithm>
-#include "gemm_f32.hpp"
+#include "gemm_split.hpp"
 #include "../../include/stade_hip.h"
 
 #include <math.h>
@@ -1099,6 +1104,13 @@ __global__ __launch_bounds__(NT) void final_kernel(FinalArgs f) {
     final_block<MODE>(f, blockIdx.x, red);
 }
 
+// resident blocks per CU of the adjoint's paired backward launch (its registers would allow
+// four; three measured faster)
+#ifndef STADE_MLP_BWD_BLOCKS
+#define STADE_MLP_BWD_BLOCKS 3
+#endif
+constexpr int kBwdBlocksPerCu = STADE_MLP_BWD_BLOCKS;
+
 // the final sums as extra blocks of the backward products' launch (they read only the head
 // and column-sum partials, so they run beside the product tiles)
 template <int MODE>
@@ -1165,11 +1177,8 @@ int32_t run(const Ptrs& p, int64_t B_, int64_t I_, int64_t H_, int64_t O_, hipSt
     // products: one launch each, operand tiles shared)
     const Plan p_s1 = plan(H, B, I, cus), p_s1d = plan(H, B, I, cus, 2);
     // (the backward products only accumulate into shadows: their K splits may add by atomics)
-    // (and they run as one launch, so with one tile width)
-    const Plan p_w1bd = plan(H, I, B, cus, 2, true), p_xbd = plan(I, B, H, cus, 2, true);
-    auto both = [&](int bnt) { return std::pair<Plan, Plan>(plan(H, I, B, cus, 1, true, bnt), plan(I, B, H, cus, 1, true, bnt)); };
-    const auto n64 = both(64), n128 = both(128);
-    const auto& [p_w1b, p_xb] = n64.first.us + n64.second.us <= n128.first.us + n128.second.us ? n64 : n128;
+    const Plan p_w1b = plan(H, I, B, cus, 1, true), p_w1bd = plan(H, I, B, cus, 2, true);
+    const Plan p_xb = plan(I, B, H, cus, 1, true), p_xbd = plan(I, B, H, cus, 2, true);
     size_t npart = 0;
     auto need = [&](const Plan& q, long M, long N) {
         if (q.ksplit > 1) npart = std::max(npart, (size_t)q.ksplit * M * N);
@@ -1284,16 +1293,20 @@ int32_t run(const Ptrs& p, int64_t B_, int64_t I_, int64_t H_, int64_t O_, hipSt
         hipError_t e;
         if (MODE == ADJ) {
             gw.nseg = gx.nseg = 1;
+            const EpiAcc ew{p.w1b, H}, ex{p.xb, I};
             STADE_TIMED("mlp_gemm_bwd", stream,
-                        e = (launch_pair<false, false, EpiAcc, true, true, EpiAcc>(gw, EpiAcc{p.w1b, H}, p_w1b, gx, EpiAcc{p.xb, I},
-                                                                                   p_xb, stream, fin)));
+                        if (!(launch_split_pair<false, false, EpiAcc, true, true, EpiAcc, false>(gw, ew, gx, ex, cus, stream, fin, e)))
+                            e = (launch_pair<false, false, EpiAcc, true, true, EpiAcc>(gw, ew, p_w1b, gx, ex, p_xb, stream, fin,
+                                                                                       kBwdBlocksPerCu)));
         } else {
             gw.seg[1] = Seg{D1d, p.xd, H, I, B};     // A1 = d1d, B1 = xd'
             gx.seg[1] = Seg{p.w1d, D1d, H, H, H};    // A1 = W1d', B1 = d1d
             gw.nseg = gx.nseg = 2;
+            const EpiAccPair ew{p.w1b, p.w1bd, H}, ex{p.xb, p.xbd, I};
             STADE_TIMED("mlp_gemm_bwd2", stream,
-                        e = (launch_pair<false, false, EpiAccPair, true, true, EpiAccPair, true>(
-                            gw, EpiAccPair{p.w1b, p.w1bd, H}, p_w1bd, gx, EpiAccPair{p.xb, p.xbd, I}, p_xbd, stream, fin)));
+                        if (!(launch_split_pair<false, false, EpiAccPair, true, true, EpiAccPair, true>(gw, ew, gx, ex, cus, stream, fin, e)))
+                            e = (launch_pair<false, false, EpiAccPair, true, true, EpiAccPair, true>(gw, ew, p_w1bd, gx, ex, p_xbd,
+                                                                                                     stream, fin)));
         }
         if (e != hipSuccess) return check_hip(e, "mlp gemm w1b + xb");
     }

@@ -46,7 +46,7 @@ def _src_key(src: str) -> str:
     flags = " ".join(f for f in FLAGS[1:] if f != str(CSRC))
     rt = (CSRC / "lowered_rt.hpp").read_text()
     if '#include "lowered_gemm.hpp"' in src:
-        rt += "".join((CSRC / h).read_text() for h in ("lowered_gemm.hpp", "gemm_f32.hpp", "split_bf16.hpp"))
+        rt += (CSRC / "lowered_gemm.hpp").read_text() + (CSRC / "gemm_f32.hpp").read_text()
     return hashlib.sha256((src + flags + rt).encode()).hexdigest()[:16]
 
 
