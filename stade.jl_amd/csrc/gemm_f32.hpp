@@ -597,6 +597,13 @@ __global__ __launch_bounds__(NT) void splitk_reduce_kernel(const float* __restri
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+// every operand 16-byte aligned with leading dimensions a multiple of 4
+inline bool operands_vec(const Args& g) {
+    bool vec = true;
+    for (int s = 0; s < g.nseg; ++s)
+        vec = vec && aligned16(g.seg[s].A) && aligned16(g.seg[s].B) && g.seg[s].lda % 4 == 0 && g.seg[s].ldb % 4 == 0;
+    return vec;
+}
 
 // Tile width and K split for an M x N x K product on `cus` compute units, from a cost model
 // in microseconds: the CU with the most blocks sets the time (blocks per CU x K steps per
@@ -611,6 +618,7 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 struct Plan {
     int bnt, ksplit;
     bool atomic;  // the slices are added into the output by atomics (an accumulate epilogue)
+    double us;    // the model's time
 };
 #ifndef STADE_GEMM_STEP_US
 #define STADE_GEMM_STEP_US 0.7
@@ -625,8 +633,7 @@ inline Plan plan(int M, int N, int Ktot, int cus, int nout = 1, bool atomic_ok =
     const double work = nout == 2 ? 2.5 : 1.0;  // block-step time relative to a single product
     const long mt = (M + BM - 1) / BM;
     const long steps = (Ktot + KT - 1) / KT;
-    Plan best{64, 1, false};
-    double best_cost = 0.0;
+    Plan best{64, 1, false, 0.0};
     // (a dual product keeps the narrow tile: with the wide one its registers allow one wave per SIMD)
     for (int bnt = 64; bnt <= (nout == 2 ? 64 : 128); bnt *= 2) {
         const long tiles = mt * ((N + bnt - 1) / bnt);
@@ -640,10 +647,7 @@ inline Plan plan(int M, int N, int Ktot, int cus, int nout = 1, bool atomic_ok =
             cost /= per_cu < 2 ? 0.75 : per_cu == 2 ? 1.0 : per_cu == 3 ? 1.08 : 1.13;
             if (ks > 1) cost += atomic_ok ? 4.0 * ks * nout * (double)M * N / (STADE_GEMM_ATOMIC_GBS * 1e3)
                                           : 8.0 * ks * nout * (double)M * N / 5e6 + 3.0;
-            if (cost < best_cost || best_cost == 0.0) {
-                best_cost = cost;
-                best = Plan{bnt, ks, atomic_ok && ks > 1};
-            }
+            if (cost < best.us || best.us == 0.0) best = Plan{bnt, ks, atomic_ok && ks > 1, cost};
         }
     }
     return best;
@@ -665,15 +669,11 @@ inline int device_cus() {
 // Launch; returns the hipError of the launch.  `part` must hold ksplit * M * N floats (DUAL:
 // twice that) when the plan splits K (ask with plan() first); it may be null otherwise.  A
 // dual product takes two segments of the same K.
-// the launch-time fields of g (split, atomic, buffer-load eligibility); vec: every operand
-// 16-byte aligned with leading dimensions a multiple of 4
+// the launch-time fields of g (split, atomic, buffer-load eligibility)
 template <bool A_KM, bool B_KM, class Epi, bool DUAL>
 hipError_t prepare(Args& g, bool& vec, const Plan& p) {
     if (DUAL && (g.nseg != 2 || g.seg[0].K != g.seg[1].K)) return hipErrorInvalidValue;
-    vec = true;
-    for (int s = 0; s < g.nseg; ++s) {
-        vec = vec && aligned16(g.seg[s].A) && aligned16(g.seg[s].B) && g.seg[s].lda % 4 == 0 && g.seg[s].ldb % 4 == 0;
-    }
+    vec = operands_vec(g);
     g.ksplit = p.ksplit;
     g.atomic = p.atomic && has_atomic<Epi>::value;
     if (p.ksplit > 1 && !g.atomic && !g.part) return hipErrorInvalidValue;

@@ -404,16 +404,12 @@ __global__ __launch_bounds__(NT, 2) void split_pair_kernel(SplitPart<A0, B0, E0>
 // the other blocks' work: about 10 TB/s of issue).  Every K slice keeps at least 8 steps.
 // nout = 2 plans a dual product (three products per step over shared loads, two outputs; its tile is
 // the narrow one).  The two products of a pair take one tile width (bnt).
-struct SplitPlan {
-    Plan p;
-    double us;  // the model's time
-};
-inline SplitPlan plan_split(int M, int N, int Ktot, int cus, int nout, int bnt) {
+inline Plan plan_split(int M, int N, int Ktot, int cus, int nout, int bnt) {
     const long mt = (M + BM - 1) / BM;
     const long steps = (Ktot + KT - 1) / KT;
     const double step_us = nout == 2 ? 1.2 : bnt == 64 ? 0.48 : 0.75;
     const long tiles = mt * ((N + bnt - 1) / bnt);
-    SplitPlan best{Plan{bnt, 1, false}, 0.0};
+    Plan best{bnt, 1, false, 0.0};
     for (int ks = 1; ks <= 16; ++ks) {
         if (ks > 1 && steps / ks < 8) break;
         const long per_cu = (tiles * ks + cus - 1) / cus;
@@ -422,7 +418,7 @@ inline SplitPlan plan_split(int M, int N, int Ktot, int cus, int nout, int bnt) 
         if (ks > 1 && per_cu > 4) break;
         double cost = (double)per_cu * st * step_us * (per_cu < 2 ? 1.5 : 1.0);
         if (ks > 1) cost += 4.0 * ks * nout * (double)M * N / 1e7;
-        if (cost < best.us || best.us == 0.0) best = SplitPlan{Plan{bnt, ks, ks > 1}, cost};
+        if (cost < best.us || best.us == 0.0) best = Plan{bnt, ks, ks > 1, cost};
     }
     return best;
 }
@@ -445,29 +441,64 @@ bool split_extents(SplitArgs& q) {
     return fits;
 }
 
+// the share of g's tiles that the fp32 form loads without a test for each element
+inline double whole_share(const Args& g, const Plan& f) {
+    if (g.seg[0].K % KT != 0 || !operands_vec(g)) return 0.0;
+    const long mt = (g.M + BM - 1) / BM, nt = (g.N + f.bnt - 1) / f.bnt;
+    return (double)(g.M / BM) * (g.N / f.bnt) / ((double)mt * nt);
+}
+
+// Whether a pair of products runs by split bf16 rather than by fp32 MFMAs with the plans f0, f1.
+// A split block carries more before its first and after its last step, and two of them share a CU
+// where three fp32 ones do; the fp32 form loses most where it tests each element that it loads.
+// So fp32 stays where its tiles are whole and the products are short.  Evaluations in fp32 / split, us:
+//   adjoint, tiles whole       512 x 256 x 256 36.2 / 37.4, 2048 x 256 x 1024 75.3 / 80.2, 2048 x 640 x 640
+//                              90.7 / 99.9, 2048 x 768 x 1024 131.6 / 136.5 (model: 67 us); 4096 x 512 x 1024
+//                              159.3 / 151.9 (86 us), 4096 x 768 x 1024 206.2 / 199.8
+//   adjoint, ragged            1000 x 500 x 700 76.3 / 73.0, 130 x 675 x 207 56.8 / 48.8, 4000 x 784 x 1000 277 / 217
+//   adjoint, a few blocks of   32 x 16 x 32 23.9 / 25.7, 64 x 16 x 64 28.1 / 29.6, 128 x 64 x 512 44.2 / 47.1,
+//   sizes in sixteens          192 x 176 x 64 48.4 / 46.4, 1920 x 32 x 64 (45 blocks) 35.4 / 33.9
+//   HVP (dual), tiles whole,   1024 x 512 x 512 120.0 / 123.0, 2048 x 512 x 512 170.9 / 173.1; 512 x 512 x 512
+//   8 steps                    (128 blocks each) 102.2 / 96.9; everything else 1.01 to 1.29 times as fast split
+inline bool split_pays(const Args& g0, const Plan& f0, const Args& g1, const Plan& f1, int cus, bool dual) {
+    auto blocks = [](const Args& g, const Plan& f) {
+        return (long)((g.M + BM - 1) / BM) * ((g.N + f.bnt - 1) / f.bnt) * f.ksplit;
+    };
+    auto steps = [](const Args& g, const Plan& f) { return ((g.seg[0].K + KT - 1) / KT + f.ksplit - 1) / f.ksplit; };
+    const long b0 = blocks(g0, f0), b1 = blocks(g1, f1);
+    const double w0 = whole_share(g0, f0), w1 = whole_share(g1, f1);
+    if (dual) return !(w0 == 1.0 && w1 == 1.0 && steps(g0, f0) <= 8 && steps(g1, f1) <= 8 && b0 >= cus && b1 >= cus);
+    if (w0 >= 0.75 && w1 >= 0.75) return f0.us + f1.us >= 80.0;
+    auto sixteens = [](const Args& g) { return operands_vec(g) && (g.M | g.N | g.seg[0].K) % KT == 0; };
+    return !(sixteens(g0) && sixteens(g1) && b0 + b1 <= 32);
+}
+
 // The pair of launch_pair by split bf16; false (and nothing launched) where the sizes or the
-// operands are not for it.  Both epilogues accumulate by atomics where K is split.
+// operands are not for it (f0, f1: the fp32 form's plans).  Both epilogues accumulate by atomics
+// where K is split.
 template <bool A0, bool B0, class E0, bool A1, bool B1, class E1, bool DUAL, class X>
-bool launch_split_pair(Args g0, E0 e0, Args g1, E1 e1, int cus, hipStream_t stream, X x, hipError_t& err) {
+bool launch_split_pair(Args g0, E0 e0, const Plan& f0, Args g1, E1 e1, const Plan& f1, int cus, hipStream_t stream, X x,
+                       hipError_t& err) {
     static_assert(has_atomic<E0>::value && has_atomic<E1>::value, "a split adds its slices by atomics");
     const int nout = DUAL ? 2 : 1;
     if (g0.M <= 0 || g0.N <= 0 || g1.M <= 0 || g1.N <= 0 || (DUAL && (g0.seg[0].K != g0.seg[1].K || g1.seg[0].K != g1.seg[1].K)))
         return false;
+    if (!split_pays(g0, f0, g1, f1, cus, DUAL)) return false;
     SplitPart<A0, B0, E0> q0{SplitArgs{g0, {0, 0}, {0, 0}}, e0, 0, 0};
     SplitPart<A1, B1, E1> q1{SplitArgs{g1, {0, 0}, {0, 0}}, e1, 0, 0};
     if (!split_extents<A0, B0, DUAL>(q0.q) || !split_extents<A1, B1, DUAL>(q1.q)) return false;
     auto both = [&](int bnt) {
-        return std::pair<SplitPlan, SplitPlan>(plan_split(g0.M, g0.N, g0.seg[0].K, cus, nout, bnt),
+        return std::pair<Plan, Plan>(plan_split(g0.M, g0.N, g0.seg[0].K, cus, nout, bnt),
                                                plan_split(g1.M, g1.N, g1.seg[0].K, cus, nout, bnt));
     };
     const auto n64 = both(64), n128 = both(128);
     const auto& [p0, p1] = DUAL || n64.first.us + n64.second.us <= n128.first.us + n128.second.us ? n64 : n128;
-    const int bnt = p0.p.bnt;
-    q0.q.g.ksplit = p0.p.ksplit; q0.q.g.atomic = p0.p.atomic;
-    q1.q.g.ksplit = p1.p.ksplit; q1.q.g.atomic = p1.p.atomic;
+    const int bnt = p0.bnt;
+    q0.q.g.ksplit = p0.ksplit; q0.q.g.atomic = p0.atomic;
+    q1.q.g.ksplit = p1.ksplit; q1.q.g.atomic = p1.atomic;
     q0.gx = (g0.M + BM - 1) / BM; q0.gy = (g0.N + bnt - 1) / bnt;
     q1.gx = (g1.M + BM - 1) / BM; q1.gy = (g1.N + bnt - 1) / bnt;
-    const long nb = (long)x.count + (long)q0.gx * q0.gy * p0.p.ksplit + (long)q1.gx * q1.gy * p1.p.ksplit;
+    const long nb = (long)x.count + (long)q0.gx * q0.gy * p0.ksplit + (long)q1.gx * q1.gy * p1.ksplit;
     if constexpr (DUAL) {
         split_pair_kernel<64, true, A0, B0, E0, A1, B1, E1, X><<<(unsigned)nb, NT, 0, stream>>>(q0, q1, x);
     } else {

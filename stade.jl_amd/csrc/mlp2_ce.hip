@@ -1295,7 +1295,7 @@ int32_t run(const Ptrs& p, int64_t B_, int64_t I_, int64_t H_, int64_t O_, hipSt
             gw.nseg = gx.nseg = 1;
             const EpiAcc ew{p.w1b, H}, ex{p.xb, I};
             STADE_TIMED("mlp_gemm_bwd", stream,
-                        if (!(launch_split_pair<false, false, EpiAcc, true, true, EpiAcc, false>(gw, ew, gx, ex, cus, stream, fin, e)))
+                        if (!(launch_split_pair<false, false, EpiAcc, true, true, EpiAcc, false>(gw, ew, p_w1b, gx, ex, p_xb, cus, stream, fin, e)))
                             e = (launch_pair<false, false, EpiAcc, true, true, EpiAcc>(gw, ew, p_w1b, gx, ex, p_xb, stream, fin,
                                                                                        kBwdBlocksPerCu)));
         } else {
@@ -1304,7 +1304,8 @@ int32_t run(const Ptrs& p, int64_t B_, int64_t I_, int64_t H_, int64_t O_, hipSt
             gw.nseg = gx.nseg = 2;
             const EpiAccPair ew{p.w1b, p.w1bd, H}, ex{p.xb, p.xbd, I};
             STADE_TIMED("mlp_gemm_bwd2", stream,
-                        if (!(launch_split_pair<false, false, EpiAccPair, true, true, EpiAccPair, true>(gw, ew, gx, ex, cus, stream, fin, e)))
+                        if (!(launch_split_pair<false, false, EpiAccPair, true, true, EpiAccPair, true>(gw, ew, p_w1bd, gx, ex, p_xbd, cus,
+                                                                                                        stream, fin, e)))
                             e = (launch_pair<false, false, EpiAccPair, true, true, EpiAccPair, true>(gw, ew, p_w1bd, gx, ex, p_xbd,
                                                                                                      stream, fin)));
         }
