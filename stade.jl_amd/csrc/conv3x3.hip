@@ -56,7 +56,7 @@ __global__ __launch_bounds__(NT) void prep_kernel(const float* __restrict__ w, i
                                                   u32x4* __restrict__ wg, int* __restrict__ flags) {
     const long nf = wf ? (long)tap_chunks(C) * 9 * 128 * ((K + 63) / 64) : 0, ng = wg ? (long)tap_chunks(K) * 9 * 128 * ((C + 63) / 64) : 0;
     const long q = (long)blockIdx.x * NT + threadIdx.x;
-    u16x2 tiny = {0xffff, 0xffff};
+    uint32_t lost = 0;
     if (q < nf + ng) {
         const bool back = q >= nf;
         const long e = back ? q - nf : q;
@@ -74,12 +74,12 @@ __global__ __launch_bounds__(NT) void prep_kernel(const float* __restrict__ w, i
             v[k] = (r < R && cin < Cin) ? (back ? w[((long)cin * C + r) * 9 + (8 - t)] : w[((long)r * C + cin) * 9 + t]) : 0.f;
         }
         u32x4 c[3];
-        split8(v, c, tiny);
+        split8(v, c, lost);
         u32x4* dst = (back ? wg : wf) + ((rc * 9 + t) * 3 * 2 + i) * 64 + lane;
 #pragma unroll
         for (int part = 0; part < 3; ++part) dst[part * 128] = c[part];
     }
-    const int any = __syncthreads_or(any_tiny(tiny));
+    const int any = __syncthreads_or(any_lost(lost));
     if (threadIdx.x == 0) flags[blockIdx.x] = any;
 }
 
@@ -290,14 +290,14 @@ __global__ __launch_bounds__(64 * TY) void tap_kernel(TapArgs a) {
                     pr[p][k][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs[p], v, soff, 0));
             }
     };
-    u16x2 tiny = {0xffff, 0xffff};
+    uint32_t lost = 0;
     auto store = [&]() {
 #pragma unroll
         for (int p = 0; p < NP; ++p)
 #pragma unroll
             for (int k = 0; k < NCELL; ++k) {
                 u32x4 c[3];
-                split8(pr[p][k], c, tiny);
+                split8(pr[p][k], c, lost);
                 if ((2 * PPL) % NTH == 0 || threadIdx.x + NTH * k < 2 * PPL)
 #pragma unroll
                     for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x4*>(lds + (p * 6 + 2 * q) * PLANE + coff[k]) = c[q];
@@ -450,7 +450,7 @@ __global__ __launch_bounds__(64 * TY) void tap_kernel(TapArgs a) {
                 for (int j = 0; j < NJ; ++j)
 #pragma unroll
                     for (int q = 0; q < 16; ++q) z = __builtin_fmaf(acc[o][i][j][q], 0.f, z);
-        bool redo = z != 0.f || any_tiny(tiny);
+        bool redo = z != 0.f || any_lost(lost);
         for (int k = threadIdx.x; k < a.nflags; k += NTH) redo = redo || a.flags[k];
         if (__syncthreads_or(redo)) {
             clear();
@@ -948,11 +948,11 @@ __global__ __launch_bounds__(NT) void wgrad_kernel(WgArgs a) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) gr[i][j] = fetch(rg, j < glim[i] ? goff[i] + (uint32_t)(S * j * 4) : kPast, soff);
     };
-    u16x2 tiny = {0xffff, 0xffff};
+    uint32_t lost = 0;
     auto store_x = [&](int i, int yy) {
         const int e = threadIdx.x + NT * i, ci = e / (S + 2), s = e - ci * (S + 2);
         u32x4 c[3];
-        split8(xr[i], c, tiny);
+        split8(xr[i], c, lost);
         if (XC % NT == 0 || e < XC)
 #pragma unroll
             for (int q = 0; q < 3; ++q) xs[yy & 3][q * XPART + s * WGP + ci] = c[q];
@@ -960,7 +960,7 @@ __global__ __launch_bounds__(NT) void wgrad_kernel(WgArgs a) {
     auto store_g = [&](int i) {
         const int e = threadIdx.x + NT * i, co = e / S, s = e - co * S;
         u32x4 c[3];
-        split8(gr[i], c, tiny);
+        split8(gr[i], c, lost);
         if (GC % NT == 0 || e < GC)
 #pragma unroll
             for (int q = 0; q < 3; ++q) gs[q * GPART + s * WGP + co] = c[q];
@@ -1046,7 +1046,7 @@ __global__ __launch_bounds__(NT) void wgrad_kernel(WgArgs a) {
     for (int t = 0; t < 9; ++t)
 #pragma unroll
         for (int q = 0; q < 16; ++q) z = __builtin_fmaf(acc[t][q], 0.f, z);
-    if (__syncthreads_or(z != 0.f || any_tiny(tiny))) {
+    if (__syncthreads_or(z != 0.f || any_lost(lost))) {
         clear();
         const int c = c0 + 32 * wa + l32, k = k0 + 32 * wb + l32;
         for (long r = lo; r < hi; ++r) {

@@ -8,7 +8,7 @@
 // The matrix cores run bf16 at 16 times the fp32 rate, so six products leave a factor of 2.7.
 // Measured with fp32 MFMAs -> split, the evaluations that hold the pair (batch 4096, 784 x 1024):
 // MLP adjoint 217 -> 190 us, HVP (dual products) 596 -> 493; HVP of 1000 x 500 x 700 168 -> 161.
-// What bounds the loop is the splitting (12 vector instructions a pair of elements, 100 a
+// What bounds the loop is the splitting (11 vector instructions a pair of elements, 92 a
 // wave and step beside 24 MFMAs) and the loads and barriers that a block's two waves a SIMD do not
 // hide wholly: without the splitting and the loads the same loop runs at 270 TFLOP/s, with them
 // at 165-180.
@@ -234,7 +234,7 @@ __device__ __forceinline__ void split_block(const SplitArgs& q, const Epi& epi, 
                 for (int r = 0; r < 16; ++r) acc[o][i][j][r] = 0.f;
     static_assert(!has_row_load<Epi>::value, "an epilogue that accumulates");
     const decltype(epi.load(0, 0)) prow[2] = {};
-    u16x2 tiny = {0xffff, 0xffff};
+    uint32_t lost = 0;
 
     // one register stage of a cell per operand: a step's loads are issued a step before it is
     // split and stored.  Loads and stores are unconditional (a step past the slice reloads a
@@ -270,11 +270,11 @@ __device__ __forceinline__ void split_block(const SplitArgs& q, const Epi& epi, 
         u32x4 c[3];
 #pragma unroll
         for (int o = 0; o < NOP; ++o) {
-            split8(va[o], c, tiny);
+            split8(va[o], c, lost);
             store_cell<A_KM, BM>(c, S + o * TA);
         }
         if (BNT == 128 || DUAL || half == 0) {
-            split8(vb, c, tiny);
+            split8(vb, c, lost);
             store_cell<B_KM, BNT>(c, S + NOP * TA + (DUAL ? half * TB : 0));
         }
     };
@@ -361,7 +361,7 @@ __device__ __forceinline__ void split_block(const SplitArgs& q, const Epi& epi, 
                 for (int j = 0; j < NJ; ++j)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) z = __builtin_fmaf(acc[o][i][j][r], 0.f, z);
-        redo = z != 0.f || any_tiny(tiny);
+        redo = z != 0.f || any_lost(lost);
     }
     if (__syncthreads_or(redo)) fp32_loop<A_KM, B_KM, BNT, DUAL>(g, m0, n0, t_begin, t_end, smem, acc);
     finish_tile<BNT, DUAL>(g, epi, acc, prow, m0 + wm, n0 + wn, bz);

@@ -181,3 +181,89 @@ def test_split_conv_few_channels(mode, outputs, size):
     for (a, _, _), want, dev in zip(args, host, case.dev):
         if a in outputs:
             assert rel_err(to_host(dev).astype(np.float64), want) <= 1e-6, a
+
+
+def _bar(n):
+    """Largest error over largest value of sums of n products, each rounded at most three times at
+    the size of a partial sum by half a unit in its last place (2^-24); such errors add up as the
+    root of their number."""
+    return np.sqrt(3 * n) * 2.0 ** -24
+
+
+def _against_64_bits(kernel, mode, shapes, ints, scales, bars, zeros=(), exact=(), int_arrays=None):
+    """One generated function, its named outputs against the 64-bit oracle; arrays in `exact`
+    hold bf16 values before their scale, and those in `zeros` are zero."""
+    lib = oracle_lib(kernel, mode, "f64")
+    args = make_args(lib, f"{kernel}_{mode}", shapes, ints, {}, "split-small", np.float32, int_arrays, None)
+    for a, kind, v in args:
+        if kind != "Af":
+            continue
+        if a in exact:
+            v.view(np.uint32)[...] &= 0xffff0000
+        v *= 0.0 if a in zeros else 1.0
+        v[...] = (v.astype(np.float64) * scales.get(a, 1.0)).astype(np.float32)
+    host = [v.astype(np.float64) if isinstance(v, np.ndarray) and v.dtype == np.float32 else v for _, _, v in args]
+    lib.call(f"{kernel}_{mode}", *host)
+    case = ParityCase(kernel, mode, args, (), "f32")
+    case.run_gpu()
+    for (a, _, _), want, dev in zip(args, host, case.dev):
+        if a in bars:
+            assert np.any(want), a
+            e = rel_err(to_host(dev).astype(np.float64), want)
+            print(f"{kernel}_{mode} {a} {e:.2e} of {bars[a]:.2e}", flush=True)
+            assert e <= bars[a], a
+
+
+# exponents of a whole operand: where the last part of the split is a subnormal (from about 2^-95
+# on), both sides of where it no longer holds all bits (2^-110), under fp32's smallest normal (2^-126),
+# and wholly under 2^-134, where every part rounds to zero
+SMALL = (-98, -106, -109, -111, -122, -130, -141)
+
+
+@pytest.mark.parametrize("e", SMALL)
+@pytest.mark.parametrize("mode", ["b", "hv"])
+def test_split_product_small_samples(mode, e):
+    """W1b = D1 x' with x near 2^e and D1 near 2^-(20 + e) (the incoming h1b)."""
+    size = (150, 40, 70, 6)
+    s = {"x": 2.0 ** e, "xd": 2.0 ** e, "h1b": 2.0 ** -(22 + e), "h1bd": 2.0 ** -(22 + e), "w1": 0.1, "w1d": 0.1, "w2": 0.2, "w2d": 0.2}
+    bars = {a: _bar(size[0]) for a in (("w1b",) if mode == "b" else ("w1b", "w1bd"))}
+    _against_64_bits("mlp2_ce", mode, _shapes(size), _ints(size), s, bars, ("w1b", "w1bd"), int_arrays=dict(lab=_labels(size)))
+
+
+@pytest.mark.parametrize("e", SMALL)
+@pytest.mark.parametrize("mode", ["b", "hv"])
+def test_split_product_small_weights(mode, e):
+    """xb = W1' D1 with W1 near 2^e and D1 near 2^-(20 + e)."""
+    size = (150, 40, 70, 6)
+    s = {"w1": 2.0 ** e, "w1d": 2.0 ** e, "h1b": 2.0 ** -(22 + e), "h1bd": 2.0 ** -(22 + e), "w2": 0.2, "w2d": 0.2}
+    bars = {a: _bar(size[2]) for a in (("xb",) if mode == "b" else ("xb", "xbd"))}
+    _against_64_bits("mlp2_ce", mode, _shapes(size), _ints(size), s, bars, ("xb", "xbd"), int_arrays=dict(lab=_labels(size)))
+
+
+@pytest.mark.parametrize("e,exact", [(e, False) for e in SMALL] + [(-115, True), (-131, True)])
+@pytest.mark.parametrize("size", [(2, 10, 17, 6, 40), (2, 18, 20, 6, 40)])
+@pytest.mark.parametrize("product", ["out by xp", "out by w", "xpb by g", "xpb by w", "wb by xp", "wb by g"])
+def test_split_conv_small(product, size, e, exact):
+    """Each product of the adjoint with one operand near 2^e and the other near 2^-(20 + e); exact:
+    bf16 values, which the split holds down to its subnormals.  (lossb = 0 where g is small or
+    large on its own: g is then outb.)"""
+    N, C, K, H, W = size
+    shapes, ints = _conv(size)
+    out, _, by = product.split()
+    other = {"out": {"xp": "w", "w": "xp"}, "xpb": {"g": "w", "w": "g"}, "wb": {"xp": "g", "g": "xp"}}[out][by]
+    name = lambda a: "outb" if a == "g" else a  # noqa: E731
+    scales = {name(by): 2.0 ** e, name(other): 2.0 ** -(22 + e)}
+    zeros = ("out", "xpb", "wb") + (("lossb",) if out != "out" else ())
+    n = {"out": 9 * C, "xpb": 9 * K, "wb": N * H * W}[out]
+    _against_64_bits("conv3x3", "b", shapes, ints, scales, {out: _bar(n)}, zeros, (name(by),) if exact else ())
+
+
+@pytest.mark.parametrize("e", SMALL)
+@pytest.mark.parametrize("size", [(2, 10, 17, 6, 40), (2, 18, 20, 6, 40)])
+@pytest.mark.parametrize("by", ["g", "w"])
+def test_split_conv_small_two_sources(by, size, e):
+    """xpb and xpbd of the HVP (two products to an element of xpbd), as above."""
+    shapes, ints = _conv(size)
+    scales = {a + s: 2.0 ** (e if a[0] == ("o" if by == "g" else "w") else -(22 + e)) for a, s in (("outb", ""), ("outb", "d"), ("w", ""), ("w", "d"))}
+    bars = {a: _bar(18 * size[2]) for a in ("xpb", "xpbd")}
+    _against_64_bits("conv3x3", "hv", shapes, ints, scales, bars, ("xpb", "xpbd", "lossb", "lossbd"))
