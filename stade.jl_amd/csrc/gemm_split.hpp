@@ -85,13 +85,16 @@ __device__ __forceinline__ uint32_t cell_offset(long ld, int r0, int rows) {
 }
 
 // a whole k step's cell by buffer loads (soff: the step's byte offset; ld4 = ld * 4).  The
-// 128-bit loads need 4-byte alignment only.
+// 128-bit loads need 4-byte alignment only.  The scalar offset never passes the buffer's end: the
+// range check compares the lane's offset with what the scalar one leaves of the buffer, and that
+// difference must not wrap (a buffer may be shorter than a step: then nothing but the lanes'
+// offsets past every buffer is loaded, at scalar offset 0).
 template <bool KMAJ>
 __device__ __forceinline__ void load_cell(float (&v)[8], __amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t soff, uint32_t ld4) {
     if constexpr (KMAJ) {
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
-            const v4f x = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, off, soff + 32u * b, 0));
+            const v4f x = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, off + 32u * b, soff, 0));
 #pragma unroll
             for (int i = 0; i < 4; ++i) v[4 * b + i] = x[i];
         }

@@ -33,9 +33,10 @@ def _ints(size):
 
 
 @pytest.mark.parametrize("mode", ["b", "d", "hv"])
-@pytest.mark.parametrize("size", [(1, 1, 1, 1), (129, 15, 65, 5), (64, 16, 128, 5), (127, 17, 129, 3), (128, 48, 64, 4),
-                                  (161, 33, 97, 2)])
+@pytest.mark.parametrize("size", [(1, 1, 1, 1), (5, 2, 3, 2), (129, 15, 65, 5), (136, 64, 128, 5), (64, 16, 128, 5),
+                                  (127, 17, 129, 3), (128, 48, 64, 4), (161, 33, 97, 2)])
 def test_split_product_edges(mode, size):
+    """Among them operands shorter than a k step's loads, and whole tiles with a partial k step."""
     print(f"mlp2_ce_{mode} {size}", flush=True)
     run_parity("mlp2_ce", mode, _shapes(size), _ints(size), precision="f32", int_arrays=dict(lab=_labels(size)),
                scales=_scales(size))
