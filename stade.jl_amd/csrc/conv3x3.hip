@@ -49,23 +49,30 @@ __host__ __device__ __forceinline__ int tap_chunks(int Cin) { return (Cin + 15) 
 // holds rows r = 64 rt + 32 i + lane % 32, input channels 16 ch + 8 (lane / 32) + 0..7 of tap t
 // (zero past the last row or channel).  Forward: cin = c, r = co, t = 3 ky + kx.  Interior of
 // xpb: cin = co, r = c, and the tap flipped (t' = 8 - t), so both products read their source
-// at (y + ky' - 1 + ...).  Each block also writes whether it met a weight that the split cannot
-// hold (flags[block]).
+// at (y + ky' - 1 + ...).  blockIdx.y runs over the forward's rtf row tiles and then those of xpb,
+// blockIdx.z over the weights and their direction, and blockIdx.x over a row tile's cells.  Each
+// block writes whether it met a weight that the split cannot hold:
+//   flags[(blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x],
+// so that a tap block asks for those of its own row tile.
 // ------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(NT) void prep_kernel(const float* __restrict__ w, int C, int K, u32x4* __restrict__ wf,
-                                                  u32x4* __restrict__ wg, int* __restrict__ flags) {
-    const long nf = wf ? (long)tap_chunks(C) * 9 * 128 * ((K + 63) / 64) : 0, ng = wg ? (long)tap_chunks(K) * 9 * 128 * ((C + 63) / 64) : 0;
-    const long q = (long)blockIdx.x * NT + threadIdx.x;
+struct PrepArgs {
+    const float* w[2];
+    u32x4* wf[2];
+    u32x4* wg[2];
+    int* flags;
+    int C, K, rtf;
+};
+__global__ __launch_bounds__(NT) void prep_kernel(PrepArgs a) {
+    const int set = blockIdx.z, C = a.C, K = a.K;
+    const bool back = (int)blockIdx.y >= a.rtf;
+    const int rt = back ? blockIdx.y - a.rtf : blockIdx.y;
+    const int Cin = back ? K : C, R = back ? C : K, chunks = tap_chunks(Cin);
+    const float* __restrict__ w = a.w[set];
+    const long q = (long)blockIdx.x * NT + threadIdx.x;  // (ch, t, i, lane) of the row tile
     uint32_t lost = 0;
-    if (q < nf + ng) {
-        const bool back = q >= nf;
-        const long e = back ? q - nf : q;
-        const int lane = (int)(e & 63), i = (int)(e >> 6) & 1;
-        const long rest = e >> 7;
-        const int t = (int)(rest % 9);
-        const long rc = rest / 9;
-        const int Cin = back ? K : C, R = back ? C : K, chunks = tap_chunks(Cin);
-        const int ch = (int)(rc % chunks), rt = (int)(rc / chunks);
+    if (q < (long)chunks * 9 * 128) {
+        const int lane = (int)(q & 63), i = (int)(q >> 6) & 1;
+        const int rest = (int)(q >> 7), t = rest % 9, ch = rest / 9;
         const int r = 64 * rt + 32 * i + (lane & 31), c0 = 16 * ch + 8 * (lane >> 5);
         float v[8];
 #pragma unroll
@@ -75,12 +82,12 @@ __global__ __launch_bounds__(NT) void prep_kernel(const float* __restrict__ w, i
         }
         u32x4 c[3];
         split8(v, c, lost);
-        u32x4* dst = (back ? wg : wf) + ((rc * 9 + t) * 3 * 2 + i) * 64 + lane;
+        u32x4* dst = (back ? a.wg : a.wf)[set] + ((((long)rt * chunks + ch) * 9 + t) * 3 * 2 + i) * 64 + lane;
 #pragma unroll
         for (int part = 0; part < 3; ++part) dst[part * 128] = c[part];
     }
     const int any = __syncthreads_or(any_lost(lost));
-    if (threadIdx.x == 0) flags[blockIdx.x] = any;
+    if (threadIdx.x == 0) a.flags[((long)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = any;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -111,8 +118,9 @@ __global__ __launch_bounds__(NT) void prep_kernel(const float* __restrict__ w, i
 // would round less often than the six products of a tap and chunk do.  One source: a tap's
 // products are summed from zero and then added to the total.  Two sources (one chunk then): the
 // five small products of all taps first, then the h h of all taps, nine roundings in all.
-// A block that meets an element which the split cannot hold forms its tile again by
-// v_mfma_f32_32x32x2_f32 with operands straight from memory.
+// A block that meets an element which the split cannot hold, among its pixels or its row tile's
+// weights, forms its tile again by v_mfma_f32_32x32x2_f32 with operands straight from memory.
+// @@CLIFF@@
 // ------------------------------------------------------------------------------------------
 constexpr int RT = 64, CC = 16;
 constexpr int WCELLS = 9 * 6 * 64;   // weight cells of a chunk and row tile
@@ -128,8 +136,9 @@ struct TapArgs {
     const float* w[2];     // the weights themselves: (r, cin, t) at w[r * wr + cin * wc + (flip ? 8 - t : t)]
     long wr, wc;
     bool flip;
-    const int* flags;      // prep_kernel's, nflags of them
-    int nflags;
+    const int* flags;      // prep_kernel's: of row tile rt, nflags at rt * nflags, and those of the
+    int nflags;            // direction fset further on
+    long fset;
     int Cin, R, Rpad, N;
     int SH, SW, ofs;      // source plane and patch origin offset
     int H, W;             // output domain
@@ -451,7 +460,9 @@ __global__ __launch_bounds__(64 * TY) void tap_kernel(TapArgs a) {
 #pragma unroll
                     for (int q = 0; q < 16; ++q) z = __builtin_fmaf(acc[o][i][j][q], 0.f, z);
         bool redo = z != 0.f || any_lost(lost);
-        for (int k = threadIdx.x; k < a.nflags; k += NTH) redo = redo || a.flags[k];
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+            for (int k = threadIdx.x; k < a.nflags; k += NTH) redo = redo || a.flags[p * a.fset + (long)rt * a.nflags + k];
         if (__syncthreads_or(redo)) {
             clear();
             for (int c0 = 0; c0 < a.Cin; c0 += 2)
@@ -1213,9 +1224,11 @@ int32_t run(const Ptrs& p, const Dims& d, hipStream_t stream) {
     const size_t cg = MODE == TAN ? 0 : (size_t)tap_chunks(d.K) * 9 * 128 * (d.Cpad / 64);
     const size_t n32 = MODE == ADJ ? 0 : up64((size_t)d.C * 9 * d.Kpad);
     const size_t nwf = cf * 12 + 2 * n32, nwg = cg * 12;
-    const int nprep = (int)((cf + cg + NT - 1) / NT);
+    // prep_kernel's grid: blocks of a row tile, row tiles
+    const int rtf = cf ? d.Kpad / 64 : 0, rtg = cg ? d.Cpad / 64 : 0;
+    const int bpt = (std::max(rtf ? tap_chunks(d.C) : 0, rtg ? tap_chunks(d.K) : 0) * 9 * 128 + NT - 1) / NT;
     const int two = MODE == ADJ ? 1 : 2;
-    const size_t nflag = up64((size_t)two * nprep);
+    const size_t nflag = up64((size_t)two * (rtf + rtg) * bpt);
     const size_t nout = up64((size_t)d.N * d.K * d.H * d.W);
     const int ctn = d.Cpad / 64, ktn = d.Kpad / 64;
     // ctn is 0 when C = 0 (no weight gradient to form)
@@ -1237,9 +1250,9 @@ int32_t run(const Ptrs& p, const Dims& d, hipStream_t stream) {
         STADE_TIMED("conv_prep", stream, (prep32_kernel<<<(unsigned)((n32 + NT - 1) / NT), NT, 0, stream>>>(p.w, p.wd, d.C, d.K, wf, wf + n32, d.Kpad)));
         STADE_LAUNCHED("conv3x3 prep32_kernel");
     }
-    for (int s = 0; s < two && nprep > 0; ++s) {
-        STADE_TIMED("conv_prep", stream, (prep_kernel<<<nprep, NT, 0, stream>>>(s ? p.wd : p.w, d.C, d.K, MODE == ADJ ? (u32x4*)wf : nullptr,
-                                                                               (u32x4*)(s ? wg1 : wg0), flags + s * nprep)));
+    if (rtf + rtg > 0) {
+        const PrepArgs a{{p.w, p.wd}, {(u32x4*)wf, nullptr}, {(u32x4*)wg0, (u32x4*)wg1}, flags, d.C, d.K, rtf};
+        STADE_TIMED("conv_prep", stream, (prep_kernel<<<dim3(bpt, rtf + rtg, two), NT, 0, stream>>>(a)));
         STADE_LAUNCHED("conv3x3 prep_kernel");
     }
     // forward: out (and outd), loss (and lossd); adjoint seeds g (and gd), outb (and outbd) reset
@@ -1248,7 +1261,7 @@ int32_t run(const Ptrs& p, const Dims& d, hipStream_t stream) {
         a.src[0] = p.xp; a.src[1] = p.xpd;
         a.wt[0] = (u32x4*)wf; a.wt32[0] = wf; a.wt32[1] = wf + n32;
         a.w[0] = p.w; a.w[1] = p.wd; a.wr = 9L * d.C; a.wc = 9; a.flip = false;
-        a.flags = flags; a.nflags = two * nprep;
+        a.flags = flags; a.nflags = bpt;
         a.Cin = d.C; a.R = d.K; a.Rpad = d.Kpad; a.N = d.N;
         a.SH = d.Hp; a.SW = d.Wp; a.ofs = 0;
         a.H = d.H; a.W = d.W;
@@ -1285,7 +1298,7 @@ int32_t run(const Ptrs& p, const Dims& d, hipStream_t stream) {
         a.src[0] = G; a.src[1] = GD;
         a.wt[0] = (u32x4*)wg0; a.wt[1] = (u32x4*)wg1;
         a.w[0] = p.w; a.w[1] = p.wd; a.wr = 9; a.wc = 9L * d.C; a.flip = true;
-        a.flags = flags; a.nflags = two * nprep;
+        a.flags = flags + (size_t)rtf * bpt; a.nflags = bpt; a.fset = (long)(rtf + rtg) * bpt;
         a.Cin = d.K; a.R = d.C; a.Rpad = d.Cpad; a.N = d.N;
         a.SH = d.H; a.SW = d.W; a.ofs = -1;
         a.H = d.H; a.W = d.W;

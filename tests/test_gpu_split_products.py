@@ -268,3 +268,38 @@ def test_split_conv_small_two_sources(by, size, e):
     scales = {a + s: 2.0 ** (e if a[0] == ("o" if by == "g" else "w") else -(22 + e)) for a, s in (("outb", ""), ("outb", "d"), ("w", ""), ("w", "d"))}
     bars = {a: _bar(18 * size[2]) for a in ("xpb", "xpbd")}
     _against_64_bits("conv3x3", "hv", shapes, ints, scales, bars, ("xpb", "xpbd", "lossb", "lossbd"))
+
+
+@pytest.mark.parametrize("row", [3, 70, 129])
+@pytest.mark.parametrize("product", ["out", "xpb", "xpbd"])
+def test_split_conv_small_row(product, row):
+    """One output row (of three row tiles) whose weights are near 2^-120, against pixels near 2^98;
+    for xpbd only the direction's: a block must notice its own row tile's, of either set."""
+    N, C, K, H, W = size = (1, 6, 131, 5, 33) if product == "out" else (1, 131, 6, 5, 33)
+    shapes, ints = _conv(size)
+    mode = "hv" if product == "xpbd" else "b"
+    lib = oracle_lib("conv3x3", mode, "f64")
+    args = make_args(lib, f"conv3x3_{mode}", shapes, ints, {}, "split-row", np.float32, None,
+                     {a: 2.0 ** 98 for a in ("xp", "outb", "outbd")} if product != "out" else {"xp": 2.0 ** 98})
+    v = {a: x for a, _, x in args}
+    for a in ("xpb", "xpbd", "out", "lossb", "lossbd") if product != "out" else ("out",):
+        if a in v:
+            v[a][...] = 0.0
+    if product != "out":
+        v["xp"] *= np.float32(2.0 ** -98)
+    pick = (lambda a: a.reshape(K, C, 9)[row]) if product == "out" else (lambda a: a.reshape(K, C, 9)[:, row])
+    for a in ("w", "wd"):
+        if a in v:
+            pick(v[a])[...] *= np.float32(0.0 if (product == "xpbd" and a == "w") else 2.0 ** -120)
+    host = [x.astype(np.float64) if isinstance(x, np.ndarray) and x.dtype == np.float32 else x for _, _, x in args]
+    lib.call(f"conv3x3_{mode}", *host)
+    case = ParityCase("conv3x3", mode, args, (), "f32")
+    print(f"conv3x3_{mode} {product} row {row}", flush=True)
+    case.run_gpu()
+    for (a, _, _), want, dev in zip(args, host, case.dev):
+        if a == product:
+            rows = lambda x: x.reshape((N, K, H, W) if product == "out" else (N, C, H + 2, W + 2))[:, row]  # noqa: E731
+            want, got = rows(want), rows(to_host(dev).astype(np.float64))
+            if product != "out":   # (the frame is border_kernel's)
+                want, got = want[:, 1:-1, 1:-1], got[:, 1:-1, 1:-1]
+            assert np.any(want) and rel_err(got, want) <= _bar(9 * (C if product == "out" else K)), a
