@@ -120,7 +120,9 @@ __global__ __launch_bounds__(NT) void prep_kernel(PrepArgs a) {
 // five small products of all taps first, then the h h of all taps, nine roundings in all.
 // A block that meets an element which the split cannot hold, among its pixels or its row tile's
 // weights, forms its tile again by v_mfma_f32_32x32x2_f32 with operands straight from memory.
-// @@CLIFF@@
+// With one such weight in a single row tile every block does: adjoint at 8 x 64 -> 64 x 256^2 2114 us,
+// 810 without (1200 with fp32 MFMAs throughout; 2336 with a tap's loads at a time); 256 -> 256
+// channels at 32^2, a weight in one of four row tiles 791 us, 275 without (434; 1076).
 // ------------------------------------------------------------------------------------------
 constexpr int RT = 64, CC = 16;
 constexpr int WCELLS = 9 * 6 * 64;   // weight cells of a chunk and row tile
@@ -465,36 +467,42 @@ __global__ __launch_bounds__(64 * TY) void tap_kernel(TapArgs a) {
             for (int k = threadIdx.x; k < a.nflags; k += NTH) redo = redo || a.flags[p * a.fset + (long)rt * a.nflags + k];
         if (__syncthreads_or(redo)) {
             clear();
-            for (int c0 = 0; c0 < a.Cin; c0 += 2)
+            // (a channel pair's nine taps are in flight together: one memory latency a pair)
+            for (int c0 = 0; c0 < a.Cin; c0 += 2) {
+                const int c = c0 + h;
+                float wf[9][NP][2], pf[9][NP][NJ];
+#pragma unroll
                 for (int t = 0; t < 9; ++t) {
-                    const int c = c0 + h, ky = t / 3, kx = t - 3 * ky;
-                    const int sy = y0 + wave + ky + a.ofs;
-                    float wf[NP][2], pf[NP][NJ];
+                    const int sy = y0 + wave + t / 3 + a.ofs;
 #pragma unroll
                     for (int p = 0; p < NP; ++p) {
 #pragma unroll
                         for (int i = 0; i < 2; ++i) {
                             const int r = rt * RT + 32 * i + l32;
-                            wf[p][i] = c < a.Cin && r < a.R ? a.w[p][r * a.wr + c * a.wc + (a.flip ? 8 - t : t)] : 0.f;
+                            wf[t][p][i] = c < a.Cin && r < a.R ? a.w[p][r * a.wr + c * a.wc + (a.flip ? 8 - t : t)] : 0.f;
                         }
 #pragma unroll
                         for (int j = 0; j < NJ; ++j) {
-                            const int sx = x0 + 32 * j + l32 + kx + a.ofs;
-                            pf[p][j] = c < a.Cin && (unsigned)sy < (unsigned)a.SH && (unsigned)sx < (unsigned)a.SW
-                                           ? a.src[p][((long)(n * a.Cin + c) * a.SH + sy) * a.SW + sx] : 0.f;
+                            const int sx = x0 + 32 * j + l32 + t % 3 + a.ofs;
+                            pf[t][p][j] = c < a.Cin && (unsigned)sy < (unsigned)a.SH && (unsigned)sx < (unsigned)a.SW
+                                              ? a.src[p][((long)(n * a.Cin + c) * a.SH + sy) * a.SW + sx] : 0.f;
                         }
                     }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int t = 0; t < 9; ++t)
 #pragma unroll
                     for (int i = 0; i < 2; ++i)
 #pragma unroll
                         for (int j = 0; j < NJ; ++j) {
-                            acc[0][i][j] = mfma(wf[0][i], pf[0][j], acc[0][i][j]);
+                            acc[0][i][j] = mfma(wf[t][0][i], pf[t][0][j], acc[0][i][j]);
                             if constexpr (NP == 2) {
-                                acc[1][i][j] = mfma(wf[1][i], pf[0][j], acc[1][i][j]);
-                                acc[1][i][j] = mfma(wf[0][i], pf[1][j], acc[1][i][j]);
+                                acc[1][i][j] = mfma(wf[t][1][i], pf[t][0][j], acc[1][i][j]);
+                                acc[1][i][j] = mfma(wf[t][0][i], pf[t][1][j], acc[1][i][j]);
                             }
                         }
-                }
+            }
         }
     }
 
@@ -858,7 +866,9 @@ __global__ __launch_bounds__(NT) void border_kernel(BorderArgs a) {
 // A row's products (24 a tap) are summed from zero and then added to the total, which rounds
 // once a row there where v_mfma_f32_32x32x2_f32 rounds every two pixels.  The next row is
 // loaded, split and stored between the MFMAs.  A block that meets an element which the split
-// cannot hold forms its sums again in fp32 with operands straight from memory.
+// cannot hold forms its sums again in fp32 with operands straight from memory (with one such
+// pixel the adjoint at 8 x 64 -> 64 x 256^2 takes 1649 us, 810 without; through LDS, without the
+// loads of the next pixels in flight, 1678).
 // Measured, us with fp32 MFMAs (tiles of 32 x 2 pixels, each row staged twice) -> split:
 // 8 x 64 -> 64 x 256^2 390 -> 235 (165 TFLOP/s; the MFMAs alone 93 at the bf16 peak).  One wave
 // a SIMD (453 registers): what the MFMAs do not hide is the LDS reads (120 of 16 bytes a wave and
@@ -1063,16 +1073,23 @@ __global__ __launch_bounds__(NT) void wgrad_kernel(WgArgs a) {
         for (long r = lo; r < hi; ++r) {
             const WgRow w(a, r, 8 * S);
             image(w);
-            for (int px = 0; px < 8 * S; px += 2) {
-                const int x = w.x0 + px + h;
-                const float gv = fetch(rg, k < a.K && x < a.W ? (uint32_t)(k * gplane + x) * 4u : kPast, (uint32_t)(w.y * a.W) * 4u);
+            // (four pixel pairs are in flight together)
+            for (int px = 0; px < 8 * S; px += 8) {
+                float gv[4], xv[4][9];
 #pragma unroll
-                for (int t = 0; t < 9; ++t) {
-                    const int xx = x + t % 3;
-                    const float xv = fetch(rx, c < a.C && xx < Wp ? (uint32_t)(c * xplane + xx) * 4u : kPast,
-                                           (uint32_t)((w.y + t / 3) * Wp) * 4u);
-                    acc[t] = mfma(xv, gv, acc[t]);
+                for (int u = 0; u < 4; ++u) {
+                    const int x = w.x0 + px + 2 * u + h;
+                    gv[u] = fetch(rg, k < a.K && x < a.W ? (uint32_t)(k * gplane + x) * 4u : kPast, (uint32_t)(w.y * a.W) * 4u);
+#pragma unroll
+                    for (int t = 0; t < 9; ++t)
+                        xv[u][t] = fetch(rx, c < a.C && x + t % 3 < Wp ? (uint32_t)(c * xplane + x + t % 3) * 4u : kPast,
+                                         (uint32_t)((w.y + t / 3) * Wp) * 4u);
                 }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int t = 0; t < 9; ++t) acc[t] = mfma(xv[u][t], gv[u], acc[t]);
             }
         }
     }
