@@ -1,9 +1,11 @@
-"""The fp32 matrix products' split-bf16 form (csrc/gemm_f32.hpp, the tap kernel of
-csrc/conv3x3.hip) at the places where it can go wrong, through the MLP and conv entry points: K of a partial step only, of whole steps only and of both,
-output tiles with one row or column past a tile's edge; operands that the split cannot hold
-(under 2^-110), whose tiles are formed again in fp32; and operands that are not finite or
-round to infinity in bf16.  The bar is the fp32 one (1e-5 normwise against the Float32 oracle,
-with the truth rule); the split's own error is at most 2^-24 of a product."""
+"""The fp32 matrix products' split-bf16 form (csrc/gemm_split.hpp: the MLP's backward pair; the tap
+and weight-gradient kernels of csrc/conv3x3.hip) at the places where it can go wrong, through the MLP
+and conv entry points: K of a partial step only, of whole steps only and of both, output tiles
+with one row or column past a tile's edge; operands that the split cannot hold (nonzero under
+2^-110), whose tiles are formed again in fp32; and operands that are not finite or round to
+infinity in bf16.  Sizes that the rules leave to fp32 MFMAs are among them.  The bar is the fp32
+one (1e-5 normwise against the Float32 oracle, with the truth rule), and, where a lost part of
+the split must show, one against 64 bits; the split's own error is at most 2^-24 of a product."""
 import numpy as np
 import pytest
 
@@ -95,12 +97,39 @@ def _conv(size):
 @pytest.mark.parametrize("mode", ["b", "d", "hv"])
 @pytest.mark.parametrize("size", [(1, 15, 63, 3, 31), (1, 16, 64, 4, 32), (2, 17, 65, 9, 65), (1, 33, 5, 8, 33), (17, 3, 64, 61, 64)])
 def test_split_conv_edges(mode, size):
-    """One past and one short of a channel chunk, a row tile, a pixel tile; the last size has
-    enough tiles for the eight-row blocks, with a partial last one."""
+    """One past and one short of a channel chunk, a row tile, a pixel tile (four-row blocks)."""
     shapes, ints = _conv(size)
     s = 1.0 / np.sqrt(9.0 * size[1])
     print(f"conv3x3_{mode} {size}", flush=True)
     run_parity("conv3x3", mode, shapes, ints, precision="f32", scales={"w": s, "wd": s})
+
+
+def _tall(cin, r, size):
+    """Whether a product with one source takes the eight-row blocks (launch_tap's rule): no fewer
+    fp32 steps than six products a tap and chunk, and a block for every CU."""
+    import torch
+    N, _, _, H, W = size
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    return (cin + 1) // 2 >= 6 * ((cin + 15) // 16) and (W + 63) // 64 * N * ((r + 63) // 64) * ((H + 7) // 8) >= cus
+
+
+@pytest.mark.parametrize("size,scale", [((17, 31, 70, 61, 65), "ordinary"), ((33, 16, 16, 61, 64), "small xp"),
+                                        ((33, 16, 16, 61, 64), "small w")])
+def test_split_conv_eight_rows(size, scale):
+    """The eight-row blocks of the adjoint's forward and of xpb, with a partial last one, ragged
+    columns, channels and row tiles; and their fp32 fallback."""
+    N, C, K, H, W = size
+    assert _tall(C, K, size) and _tall(K, C, size)
+    shapes, ints = _conv(size)
+    s = 1.0 / np.sqrt(9.0 * C)
+    scales = {"w": s, "xp": 1.0}
+    if scale != "ordinary":
+        small, big = ("xp", "w") if scale == "small xp" else ("w", "xp")
+        scales[small] *= 2.0 ** -122
+        scales[big] *= 2.0 ** 110
+        scales["out"] = scales["outb"] = 2.0 ** -12
+    print(f"conv3x3_b {size} {scale}", flush=True)
+    run_parity("conv3x3", "b", shapes, ints, precision="f32", scales=scales)
 
 
 @pytest.mark.parametrize("mode", ["b", "hv"])
@@ -213,6 +242,16 @@ def _against_64_bits(kernel, mode, shapes, ints, scales, bars, zeros=(), exact=(
             e = rel_err(to_host(dev).astype(np.float64), want)
             print(f"{kernel}_{mode} {a} {e:.2e} of {bars[a]:.2e}", flush=True)
             assert e <= bars[a], a
+
+
+@pytest.mark.parametrize("mode", ["b", "hv"])
+def test_split_product_against_64_bits(mode):
+    """W1b and xb at K = 784: the split's own error, the rounding of a total a k step and that of D1
+    give 1 to 2e-7; without the products l h, h l and m m it would be 4e-6."""
+    size = (784, 70, 784, 5)
+    s = _scales(size)
+    bars = {a: 5e-7 for a in (("w1b", "xb") if mode == "b" else ("w1b", "xb", "w1bd", "xbd"))}
+    _against_64_bits("mlp2_ce", mode, _shapes(size), _ints(size), s, bars, ("w1b", "xb", "w1bd", "xbd"), int_arrays=dict(lab=_labels(size)))
 
 
 # exponents of a whole operand: where the last part of the split is a subnormal (from about 2^-95
