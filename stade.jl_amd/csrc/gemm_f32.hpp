@@ -228,93 +228,6 @@ constexpr int smem_floats() {
     return 2 * (DUAL ? 2 : 1) * KQ * (ldq<BM>() + ldq<BNT>());
 }
 
-// The outputs of a wave's part of a tile (rows m0.., columns n0..) of slice bz: added by atomics or
-// kept as partial sums where K is split, otherwise through the epilogue.  Accumulator (i, j, r):
-// m = m0 + 32 i + lane % 32,  n = n0 + 32 j + 8 (r / 4) + 4 (lane / 32) + r % 4
-template <int BNT, bool DUAL, class Epi, class Pre>
-__device__ __forceinline__ void finish_tile(const Args& g, const Epi& epi, const floatx16 (&acc)[DUAL ? 2 : 1][2][BNT / 64],
-                                            const Pre (&prow)[2], int m0, int n0, int bz) {
-    constexpr int NJ = BNT / 64, NOP = DUAL ? 2 : 1;
-    const int lane = threadIdx.x & 63;
-    if constexpr (has_atomic<Epi>::value) {
-        if (g.ksplit > 1 && g.atomic) {
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int m = m0 + i * 32 + (lane & 31);
-                if (m >= g.M) continue;
-#pragma unroll
-                for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int n = n0 + j * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-                        if (n < g.N) {
-                            if constexpr (DUAL)
-                                epi.atomic(m, n, acc[0][i][j][r], acc[NOP - 1][i][j][r]);
-                            else
-                                epi.atomic(m, n, acc[0][i][j][r]);
-                        }
-                    }
-            }
-            return;
-        }
-    }
-    if (g.ksplit > 1) {
-        // slice z at part + z * NOP * M * N (DUAL: P then Q)
-        const long mn = (long)g.M * g.N;
-        float* part = g.part + (long)bz * NOP * mn;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int m = m0 + i * 32 + (lane & 31);
-            if (m >= g.M) continue;
-#pragma unroll
-            for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int n = n0 + j * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-                    if (n < g.N) {
-#pragma unroll
-                        for (int o = 0; o < NOP; ++o) part[o * mn + m + (long)n * g.M] = acc[o][i][j][r];
-                    }
-                }
-        }
-        return;
-    }
-    // the epilogue's inputs (e.g. C of C += v) for the whole tile first, then the stores: the
-    // output may alias them as far as the compiler knows, and interleaving would serialise one
-    // memory round trip per element
-    Pre pre[2][NJ][16];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = m0 + i * 32 + (lane & 31);
-                const int n = n0 + j * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-                if constexpr (has_row_load<Epi>::value)
-                    pre[i][j][r] = prow[i];
-                else
-                    pre[i][j][r] = (m < g.M && n < g.N) ? epi.load(m, n) : Pre{};
-            }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int m = m0 + i * 32 + (lane & 31);
-        if (m >= g.M) continue;
-#pragma unroll
-        for (int j = 0; j < NJ; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int n = n0 + j * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-                if (n < g.N) {
-                    if constexpr (DUAL)
-                        epi(m, n, acc[0][i][j][r], acc[NOP - 1][i][j][r], pre[i][j][r]);
-                    else
-                        epi(m, n, acc[0][i][j][r], pre[i][j][r]);
-                }
-            }
-    }
-}
-
 // One block of the product: the tile at (bx, by) of slice bz, with its LDS at smem.
 template <bool A_KM, bool B_KM, int BNT, class Epi, bool DUAL>
 __device__ __forceinline__ void gemm_block(const Args& g, bool vec, const Epi& epi, int bx, int by, int bz, float* smem) {
@@ -511,7 +424,84 @@ __device__ __forceinline__ void gemm_block(const Args& g, bool vec, const Epi& e
     };
     if (full) mainloop(std::true_type{});
     else mainloop(std::false_type{});
-    finish_tile<BNT, DUAL>(g, epi, acc, prow, m0 + wm, n0 + wn, bz);
+    // accumulator (i, j, r): m = m0 + wm + 32 i + lane % 32,  n = n0 + wn + 32 j + 8 (r / 4) + 4 (lane / 32) + r % 4
+    if constexpr (has_atomic<Epi>::value) {
+        if (g.ksplit > 1 && g.atomic) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int m = m0 + wm + i * 32 + (lane & 31);
+                if (m >= g.M) continue;
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int n = n0 + wn + j * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
+                        if (n < g.N) {
+                            if constexpr (DUAL)
+                                epi.atomic(m, n, acc[0][i][j][r], acc[NOP - 1][i][j][r]);
+                            else
+                                epi.atomic(m, n, acc[0][i][j][r]);
+                        }
+                    }
+            }
+            return;
+        }
+    }
+    if (g.ksplit > 1) {
+        // slice z at part + z * NOP * M * N (DUAL: P then Q)
+        const long mn = (long)g.M * g.N;
+        float* part = g.part + (long)bz * NOP * mn;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int m = m0 + wm + i * 32 + (lane & 31);
+            if (m >= g.M) continue;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int n = n0 + wn + j * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
+                    if (n < g.N) {
+#pragma unroll
+                        for (int o = 0; o < NOP; ++o) part[o * mn + m + (long)n * g.M] = acc[o][i][j][r];
+                    }
+                }
+        }
+        return;
+    }
+    // the epilogue's inputs (e.g. C of C += v) for the whole tile first, then the stores: the
+    // output may alias them as far as the compiler knows, and interleaving would serialise one
+    // memory round trip per element
+    Pre pre[2][NJ][16];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m = m0 + wm + i * 32 + (lane & 31);
+                const int n = n0 + wn + j * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
+                if constexpr (has_row_load<Epi>::value)
+                    pre[i][j][r] = prow[i];
+                else
+                    pre[i][j][r] = (m < g.M && n < g.N) ? epi.load(m, n) : Pre{};
+            }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int m = m0 + wm + i * 32 + (lane & 31);
+        if (m >= g.M) continue;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int n = n0 + wn + j * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
+                if (n < g.N) {
+                    if constexpr (DUAL)
+                        epi(m, n, acc[0][i][j][r], acc[NOP - 1][i][j][r], pre[i][j][r]);
+                    else
+                        epi(m, n, acc[0][i][j][r], pre[i][j][r]);
+                }
+            }
+    }
 }
 
 template <bool A_KM, bool B_KM, int BNT, class Epi, bool DUAL = false>

@@ -196,7 +196,8 @@ __device__ __forceinline__ void fp32_loop(const Args& g, int m0, int n0, int t_b
     }
 }
 
-// One block of the product: the tile at (bx, by) of slice bz, with its LDS at smem.
+// One block of the product: the tile at (bx, by) of slice bz, with its LDS at smem.  The epilogue
+// accumulates into its output, by atomics where K is split.
 template <bool A_KM, bool B_KM, int BNT, class Epi, bool DUAL>
 __device__ __forceinline__ void split_block(const SplitArgs& q, const Epi& epi, int bx, int by, int bz, float* smem) {
     const Args& g = q.g;
@@ -235,8 +236,6 @@ __device__ __forceinline__ void split_block(const SplitArgs& q, const Epi& epi, 
             for (int j = 0; j < NJ; ++j)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[o][i][j][r] = 0.f;
-    static_assert(!has_row_load<Epi>::value, "an epilogue that accumulates");
-    const decltype(epi.load(0, 0)) prow[2] = {};
     uint32_t lost = 0;
 
     // one register stage of a cell per operand: a step's loads are issued a step before it is
@@ -367,7 +366,36 @@ __device__ __forceinline__ void split_block(const SplitArgs& q, const Epi& epi, 
         redo = z != 0.f || any_lost(lost);
     }
     if (__syncthreads_or(redo)) fp32_loop<A_KM, B_KM, BNT, DUAL>(g, m0, n0, t_begin, t_end, smem, acc);
-    finish_tile<BNT, DUAL>(g, epi, acc, prow, m0 + wm, n0 + wn, bz);
+    // accumulator (i, j, r): m = m0 + wm + 32 i + lane % 32,  n = n0 + wn + 32 j + 8 (r / 4) + 4 (lane / 32) + r % 4
+    auto each = [&](auto&& f) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int m = m0 + wm + i * 32 + (lane & 31);
+            if (m >= g.M) continue;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int n = n0 + wn + j * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
+                    if (n < g.N) f(i, j, r, m, n);
+                }
+        }
+    };
+    if (g.ksplit > 1) {
+        each([&](int i, int j, int r, int m, int n) {
+            if constexpr (DUAL) epi.atomic(m, n, acc[0][i][j][r], acc[1][i][j][r]);
+            else epi.atomic(m, n, acc[0][i][j][r]);
+        });
+        return;
+    }
+    // the old values of the whole tile first, then the stores: the output may alias them as far
+    // as the compiler knows, and interleaving would serialise one memory round trip per element
+    decltype(epi.load(0, 0)) pre[2][NJ][16];
+    each([&](int i, int j, int r, int m, int n) { pre[i][j][r] = epi.load(m, n); });
+    each([&](int i, int j, int r, int m, int n) {
+        if constexpr (DUAL) epi(m, n, acc[0][i][j][r], acc[1][i][j][r], pre[i][j][r]);
+        else epi(m, n, acc[0][i][j][r], pre[i][j][r]);
+    });
 }
 
 // Two products in one launch, as gemm_pair_kernel
@@ -497,8 +525,8 @@ bool launch_split_pair(Args g0, E0 e0, const Plan& f0, Args g1, E1 e1, const Pla
     const auto n64 = both(64), n128 = both(128);
     const auto& [p0, p1] = DUAL || n64.first.us + n64.second.us <= n128.first.us + n128.second.us ? n64 : n128;
     const int bnt = p0.bnt;
-    q0.q.g.ksplit = p0.ksplit; q0.q.g.atomic = p0.atomic;
-    q1.q.g.ksplit = p1.ksplit; q1.q.g.atomic = p1.atomic;
+    q0.q.g.ksplit = p0.ksplit;
+    q1.q.g.ksplit = p1.ksplit;
     q0.gx = (g0.M + BM - 1) / BM; q0.gy = (g0.N + bnt - 1) / bnt;
     q1.gx = (g1.M + BM - 1) / BM; q1.gy = (g1.N + bnt - 1) / bnt;
     const long nb = (long)x.count + (long)q0.gx * q0.gy * p0.ksplit + (long)q1.gx * q1.gy * p1.ksplit;
