@@ -349,9 +349,10 @@ __global__ __launch_bounds__(NT) void zero2_kernel(double* __restrict__ a, doubl
 // the last strip and the last chunk are then moved back to end at n, and their columns and rows
 // that the strip or chunk before owns are computed again but neither stored nor summed.  Loads
 // stay unconditional.  Against the row-streaming kernels, which reload three to five rows per
-// row out of LDS behind a barrier (tangent / adjoint / HVP, us): n = 100 24 -> 13 / 35 -> 14 /
-// 52 -> 19, n = 1000 28 -> 15 / 41 -> 20 / 60 -> 34, n = 3000 72 -> 65 / 101 -> 78 / 207 -> 184,
-// n = 5000 179 -> 158 / 260 -> 219 / 520 -> 438.
+// row out of LDS behind a barrier (tangent / adjoint / HVP, us, on the same arrays each time): n = 100
+// 24 -> 12 / 35 -> 15 / 53 -> 20, n = 1000 28 -> 15 / 41 -> 20 / 60 -> 32, n = 3000 64 -> 54 /
+// 85 -> 78 / 205 -> 165 (tangent on arrays that no cache holds 74 -> 71), n = 5000 180 -> 151 /
+// 259 -> 209 / 522 -> 438.
 //
 // One wavefront owns a strip of 64 columns (lane l: column c0 + l) and a chunk of WCH rows,
 // and marches down it alone: no LDS, no barriers.  East / west neighbours come from the
@@ -886,7 +887,8 @@ bool wave_path(int64_t n) { return n >= WS && (n % WS == 0 || n <= kRaggedMax); 
 // rows of a 64-column strip's chunk at ragged sizes: 16 rows for the waves that a smaller grid
 // needs, 32 from where the grid fills the chip with those (fewer halo rows, half the partials).
 // Adjoint, 16 against 32 rows: n = 1001 18.3 / 21.4 us, 3001 99 / 101, 4095 181 / 177,
-// 7001 533 / 517 (the row-streaming kernels: 40.8, 104, 179, 528)
+// 7001 533 / 517 (the row-streaming kernels in the same run: 40.8, 104, 179, 528; in another,
+// this rule against them: 1001 17.9 / 40.7, 3001 86.8 / 86.6, 4095 168 / 174)
 int rows_ragged(int64_t n) { return n < 3584 ? 16 : 32; }
 WaveGrid wave_grid64(int64_t n, int rows) { return wave_grid(n, WS, n % WS == 0 ? rows : rows_ragged(n)); }
 // calls f with whether the strips are ragged as a compile-time constant

@@ -7,8 +7,8 @@
 // v_mfma_f32_32x32x2_f32 5.0e-7 and 1.1e-6, accumulated straight 4.0e-7 and 9.9e-7.
 // The matrix cores run bf16 at 16 times the fp32 rate, so six products leave a factor of 2.7.
 // Measured with fp32 MFMAs -> split, the evaluations that hold the pair (batch 4096, 784 x 1024):
-// MLP adjoint 217 -> 190 us, HVP (dual products) 596 -> 493; HVP of 1000 x 500 x 700 168 -> 161.
-// What bounds the loop is the splitting (11 vector instructions a pair of elements, 92 a
+// MLP adjoint 208 -> 179 us, HVP (dual products) 595 -> 479; HVP of 1000 x 500 x 700 168 -> 160.
+// What bounds the loop is the splitting (12 vector instructions a pair of elements, 96 a
 // wave and step beside 24 MFMAs) and the loads and barriers that a block's two waves a SIMD do not
 // hide wholly: without the splitting and the loads the same loop runs at 270 TFLOP/s, with them
 // at 165-180.
@@ -482,15 +482,16 @@ inline double whole_share(const Args& g, const Plan& f) {
 // Whether a pair of products runs by split bf16 rather than by fp32 MFMAs with the plans f0, f1.
 // A split block carries more before its first and after its last step, and two of them share a CU
 // where three fp32 ones do; the fp32 form loses most where it tests each element that it loads.
-// So fp32 stays where its tiles are whole and the products are short.  Evaluations in fp32 / split, us:
-//   adjoint, tiles whole       512 x 256 x 256 36.2 / 37.4, 2048 x 256 x 1024 75.3 / 80.2, 2048 x 640 x 640
-//                              90.7 / 99.9, 2048 x 768 x 1024 131.6 / 136.5 (model: 67 us); 4096 x 512 x 1024
-//                              159.3 / 151.9 (86 us), 4096 x 768 x 1024 206.2 / 199.8
-//   adjoint, ragged            1000 x 500 x 700 76.3 / 73.0, 130 x 675 x 207 56.8 / 48.8, 4000 x 784 x 1000 277 / 217
-//   adjoint, a few blocks of   32 x 16 x 32 23.9 / 25.7, 64 x 16 x 64 28.1 / 29.6, 128 x 64 x 512 44.2 / 47.1,
-//   sizes in sixteens          192 x 176 x 64 48.4 / 46.4, 1920 x 32 x 64 (45 blocks) 35.4 / 33.9
-//   HVP (dual), tiles whole,   1024 x 512 x 512 120.0 / 123.0, 2048 x 512 x 512 170.9 / 173.1; 512 x 512 x 512
-//   8 steps                    (128 blocks each) 102.2 / 96.9; everything else 1.01 to 1.29 times as fast split
+// So fp32 stays where its tiles are whole and the products are short, and for a few blocks that
+// test nothing, where either form may be the faster.  Evaluations in fp32 / split, us:
+//   adjoint, tiles whole       512 x 256 x 256 36.7 / 36.4, 2048 x 256 x 1024 75.7 / 80.2, 2048 x 640 x 640
+//                              90.8 / 99.7, 2048 x 768 x 1024 131.7 / 137.7 (model: 67 us); 4096 x 512 x 1024
+//                              157.6 / 152.0 (86 us), 4096 x 768 x 1024 219.3 / 204.8
+//   adjoint, ragged            1000 x 500 x 700 76.4 / 72.6, 130 x 675 x 207 56.8 / 48.8, 4000 x 784 x 1000 282 / 218
+//   adjoint, a few blocks of   384 x 144 x 192 42.3 / 43.8, 128 x 64 x 512 44.2 / 44.9, 32 x 16 x 32 25.6 / 24.4,
+//   sizes in sixteens          192 x 176 x 64 48.2 / 45.0; with 45 blocks 1920 x 32 x 64 35.4 / 32.9
+//   HVP (dual), tiles whole,   1024 x 512 x 512 119.7 / 124.8, 2048 x 512 x 512 171.4 / 174.6; 512 x 512 x 512
+//   8 steps                    (128 blocks each) 101.7 / 97.3; everything else 1.01 to 1.3 times as fast split
 inline bool split_pays(const Args& g0, const Plan& f0, const Args& g1, const Plan& f1, int cus, bool dual) {
     auto blocks = [](const Args& g, const Plan& f) {
         return (long)((g.M + BM - 1) / BM) * ((g.N + f.bnt - 1) / f.bnt) * f.ksplit;
