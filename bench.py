@@ -38,7 +38,8 @@ for _p in (ROOT, ROOT / "stade.jl_amd"):
 HBM_PEAK_GBS = 8000.0
 FP32_PEAK_TFLOPS = 157.3
 FP64_PEAK_TFLOPS = 78.6
-# fp32 products by split bf16 are six bf16 products each (2.5 PFLOP/s dense)
+# fp32 products by split bf16 are six bf16 products each (2.5 PFLOP/s dense); which launches run
+# so at the benchmark's sizes (small MLP pairs stay on fp32 MFMAs)
 SPLIT_PEAK_TFLOPS = 2500.0 / 6.0
 SPLIT_KERNELS = {"mlp_gemm_bwd", "mlp_gemm_bwd2", "conv_fwd", "conv_wgrad", "conv_wgrad2", "conv_dgrad", "conv_dgrad_hv"}
 

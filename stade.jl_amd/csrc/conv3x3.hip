@@ -109,11 +109,11 @@ __global__ __launch_bounds__(NT) void prep_kernel(PrepArgs a) {
 // weights (two sets, too many for LDS) from the cache.  The two outputs' sums are kept per chunk
 // and then added to their totals, which more than halves their rounding.
 // Measured, us with fp32 MFMAs -> split: 8 x 64 -> 64 x 256^2, forward 391 -> 287, xpb 385 -> 270;
-// the matrix cores are busy for 40 % of it.  Without the MFMAs' operands being staged, the
+// the matrix cores are busy for 38 and 39 % of it.  Without the MFMAs' operands being staged, the
 // MFMAs and the epilogue alone take 186 and 157 us (672 and 406 MB of HBM traffic); weights
 // from the cache with four rows a block: 306 and 290; the splitting interleaved with the MFMAs
-// over a double-buffered patch: no faster.  Error against 64 bits 5.0e-7 -> 4.2e-7 (one source),
-// 3.0e-7 -> 1.8e-7 (two).
+// over a double-buffered patch: no faster.  Error against 64 bits 5.0e-7 -> 4.2e-7 (one source;
+// two: xpb 3.8e-7 -> 2.3e-7, xpbd 6.4e-7 -> 4.4e-7 at 4 x 32 -> 48 x 112 x 100).
 // FRESH: fewer roundings at the total's size, for few channels, where v_mfma_f32_32x32x2_f32
 // would round less often than the six products of a tap and chunk do.  One source: a tap's
 // products are summed from zero and then added to the total.  Two sources (one chunk then): the
