@@ -9,12 +9,8 @@
 // (`cgen_adjoint_contraction_` 14762) are CUDA-only.
 //
 // Here the three contractions run on the matrix cores, each with its elementwise neighbours fused
-// into the epilogue: the forward by fp32 MFMAs (gemm_f32.hpp), the backward pair by split bf16
-// (gemm_split.hpp).  By split bf16 the adjoint's forward takes as long (4096 x 784 -> 1024: 70 us) and
-// the tangent's dual one less (179 -> 121 us), but the sums over the batch that follow are then
-// further from 64 bits (b2b at 1000 x 500 x 700 3.1e-8 -> 5.8e-8, w2b 7.2e-8 -> 9.0e-8, b1b 6.0e-8 ->
-// 7.6e-8, rms over 30 seeds), and lossd, whose terms cancel, moves by more than 5e-6 in 1 of 30
-// draws:
+// into the epilogue; the forward by fp32 MFMAs (gemm_f32.hpp), the backward pair by split bf16 where
+// that is the faster form (gemm_split.hpp):
 //   S1 = W1 X            epilogue h1 = tanh(S1 + b1)                 (H x B, K = I)
 //   head (per sample)    z = W2 h1 + b2, CE, d2 = dloss/dz, zb reset,
 //                        d1 = (1 - h1^2) (h1b + W2' d2), h1b reset    (one wave per sample)
@@ -24,6 +20,12 @@
 // The adjoint (i_h <= 1024) forms head and column sums in one pass over h1 (headd1_kernel);
 // the tangent adds S1d = W1d X + W1 Xd (one dual GEMM, epilogue h1d = (1 - h1^2)(S1d + b1d));
 // the HVP adds the tangents of every backward product in dual launches.
+//
+// Why the forward is not split: the adjoint's takes as long either way (4096 x 784 -> 1024: 70 us) and
+// the tangent's dual one less (179 -> 121 us), but what is summed from it loses.  lossd, whose terms
+// cancel, moves by more than 5e-6 for 1 in 30 inputs, and the sums over the batch are further
+// from 64 bits (rms over 30 seeds at 1000 x 500 x 700: b2b 3.1e-8 -> 5.8e-8, w2b 7.2e-8 -> 9.0e-8, b1b
+// 6.0e-8 -> 7.6e-8).
 #include "internal.hpp"
 
 #include <algorithm>
